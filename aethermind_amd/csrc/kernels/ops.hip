@@ -192,9 +192,11 @@ __global__ __launch_bounds__(256) void fill_kernel(typename A::T* out, int64_t n
 }
 
 // ---------------- Argmax ----------------
-// grid (blocks_per_row, rows).  Each block reduces a slice, writes (value, index)
-// to the workspace; the last block of a row (atomic ticket) reduces the partials
-// and resets the ticket to zero for the next call.
+// grid (blocks_per_row, rows).  Each block reduces a slice in 16-byte loads, writes
+// (value, index) to the workspace; the last block of a row (atomic ticket) reduces the
+// partials, one per thread, and resets the ticket to zero for the next call.
+// Latency-bound: four fp32 rows of 128,256 took 19.8 us while one thread of the last
+// block read the 63 partials one after the other; with all of them in flight 7.6 us.
 struct ArgmaxWs {
   static constexpr int kMaxBlocks = 64;
 };
@@ -210,34 +212,57 @@ __global__ __launch_bounds__(256) void argmax_kernel(const typename A::T* x, int
   const typename A::T* row = x + r * n;
   float bv = 0.0f;
   int64_t bi = -1;
-  for (int64_t j = blockIdx.x * 256 + threadIdx.x; j < n; j += static_cast<int64_t>(nb) * 256) {
+  constexpr int V = 16 / sizeof(typename A::T);  // values per 16-byte load
+  const int64_t step = static_cast<int64_t>(nb) * 256;
+  const int64_t nv = (reinterpret_cast<uintptr_t>(row) & 15u) == 0 ? n / V : 0;  // whole aligned vectors
+  for (int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; c < nv; c += step) {
+    const uint4 raw = reinterpret_cast<const uint4*>(row)[c];
+    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      float v;
+      if constexpr (V == 4) v = __uint_as_float(w[e]);
+      else v = bf16_bits_to_f32((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xFFFFu));
+      if (argmax_better(v, c * V + e, bv, bi)) {
+        bv = v;
+        bi = c * V + e;
+      }
+    }
+  }
+  for (int64_t j = nv * V + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; j < n; j += step) {
     const float v = A::load(row, j);
     if (argmax_better(v, j, bv, bi)) {
       bv = v;
       bi = j;
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o, 64);
-    const int64_t oi = __shfl_xor(bi, o, 64);
-    if (oi >= 0 && argmax_better(ov, oi, bv, bi)) {
-      bv = ov;
-      bi = oi;
-    }
-  }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-    sv[wave] = bv;
-    si[wave] = bi;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 4; ++w)
-      if (si[w] >= 0 && argmax_better(sv[w], si[w], bv, bi)) {
-        bv = sv[w];
-        bi = si[w];
+  // best of the block (sv, si hold a pair per wave), in thread 0
+  auto block_best = [&]() {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const float ov = __shfl_xor(bv, o, 64);
+      const int64_t oi = __shfl_xor(bi, o, 64);
+      if (oi >= 0 && argmax_better(ov, oi, bv, bi)) {
+        bv = ov;
+        bi = oi;
       }
+    }
+    if (lane == 0) {
+      sv[wave] = bv;
+      si[wave] = bi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 1; w < 4; ++w)
+        if (si[w] >= 0 && argmax_better(sv[w], si[w], bv, bi)) {
+          bv = sv[w];
+          bi = si[w];
+        }
+    }
+  };
+  block_best();
+  if (threadIdx.x == 0) {
     // device-coherent (sc1) stores, acknowledged before the relaxed ticket: the last
     // block's device-coherent loads then see every block's partial
     __hip_atomic_store(&pv[r * ArgmaxWs::kMaxBlocks + blockIdx.x], bv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -247,20 +272,18 @@ __global__ __launch_bounds__(256) void argmax_kernel(const typename A::T* x, int
     last = (t == static_cast<unsigned>(nb - 1));
   }
   __syncthreads();
-  if (last && threadIdx.x == 0) {
-    float fv = 0.0f;
-    int64_t fi = -1;
-    for (int b = 0; b < nb; ++b) {
-      const float v = __hip_atomic_load(&pv[r * ArgmaxWs::kMaxBlocks + b], __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-      const int64_t i = __hip_atomic_load(&pi[r * ArgmaxWs::kMaxBlocks + b], __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT);
-      if (i >= 0 && argmax_better(v, i, fv, fi)) {
-        fv = v;
-        fi = i;
-      }
-    }
-    out[r] = fi < 0 ? 0 : fi;
+  if (!last) return;
+  // one partial per thread: every device-coherent load is in flight at once
+  static_assert(ArgmaxWs::kMaxBlocks <= 256, "one partial per thread");
+  bv = 0.0f;
+  bi = -1;
+  if (static_cast<int>(threadIdx.x) < nb) {
+    bv = __hip_atomic_load(&pv[r * ArgmaxWs::kMaxBlocks + threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bi = __hip_atomic_load(&pi[r * ArgmaxWs::kMaxBlocks + threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  block_best();
+  if (threadIdx.x == 0) {
+    out[r] = bi < 0 ? 0 : bi;
     tickets[r] = 0u;
   }
 }
