@@ -91,6 +91,12 @@ am_status_code GemmI4(const void* x, int64_t m, const am_gfx950_weight& w, int32
 am_status_code GemmI4QkvRopeKv(const void* x, int64_t m, const am_gfx950_weight& w, const am_gfx950_prefill_rope_kv& r,
                                void* q_out, void* ws, int64_t ws_bytes, hipStream_t s);
 
+// fp32 Linear for two or more rows (gemm_f32.hip), for the row lengths and residuals the
+// fp32 GEMV accepts.
+bool GemmF32Eligible(const am_gfx950_weight& w, int64_t m, const void* x, const void* residual);
+am_status_code GemmF32(const void* x, int64_t m, const am_gfx950_weight& w, void* out, const void* residual,
+                       hipStream_t s);
+
 // ---- device: numeric helpers ----
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
 

@@ -421,7 +421,10 @@ extern "C" am_status_code am_gfx950_linear(const am_gfx950_linear_args* a, void*
     AM_RETURN_IF_LAUNCH_FAILED("gemm");
     return AM_STATUS_OK;
   }
-  // GEMV per row (decode, fp32 activations, or shapes the GEMM does not tile).
+  if (a->mode == 0 && a->x_dtype == AM_DT_F32 && GemmF32Eligible(w, a->m, a->x, a->residual))
+    return GemmF32(a->x, a->m, w, a->out, a->residual, s);
+  // GEMV per row (decode, fp32 activations with other weights, or shapes the GEMMs do
+  // not tile).
   const int64_t esz = a->x_dtype == AM_DT_F32 ? 4 : 2;
   const int64_t osz = a->out_dtype == AM_DT_F32 ? 4 : 2;
   for (int64_t r = 0; r < a->m; ++r) {
