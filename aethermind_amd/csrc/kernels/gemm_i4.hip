@@ -2,33 +2,37 @@
 // (v_mfma_f32_16x16x32_bf16) for INT4 g128, INT8 per-channel and bf16 weights, with the
 // prefill plan's fused epilogues.
 //
-//   * Block tile 128 x 128 (M x N), k step 64, 256 threads = 2 x 2 waves of 64 x 64
-//     (4 x 4 MFMA tiles each), or 128 x 256 with 8 waves when that still gives every
-//     CU a tile.
+//   * Block tiles from 64 x 64 to 256 x 256 (TileCfg), chosen per launch by an estimate
+//     of its time (EstimateUs).  What bounds them: few rows, the weight stream and the
+//     first loads' latency; many rows, the matrix pipe, which the LDS reads, the weight
+//     conversions and the barriers of the k loop have to stay behind.
 //   * Operands move global -> LDS by DMA (global_load_lds_dwordx4): no registers and no
-//     LDS store instructions, so two or three k steps are in flight while one is
-//     computed.  The ring holds the stages of X (128 rows x 128 B) and W (rows of 32 B
-//     INT4, 64 B INT8 or 128 B bf16 per k step), plus for INT4 a four-slot ring of the
-//     fp16 group scales.
+//     LDS store instructions, so two or more k steps are in flight while one is
+//     computed.  The ring holds the stages of X and W (per 64 k values, 128 bytes of an X
+//     row and 32 B INT4, 64 B INT8 or 128 B bf16 of a W row), plus for INT4 a four-slot
+//     ring of the fp16 group scales.
 //   * DMA writes a wave's 64 lanes to 1 KB of consecutive LDS, so the bank layout is
-//     set by which global chunk each lane fetches: 16-byte chunk c of X row r (and of a
-//     bf16 W row) sits at slot c ^ ((r >> 1) & 7) of the row, chunk c of an INT8 W row n
-//     at slot c ^ ((n >> 2) & 3), chunk c of an INT4 W row n at slot c ^ ((n >> 3) & 1).
-//     The 16 rows read by one MFMA operand fetch then fall into distinct banks.
-//   * The weight stays in its storage format in LDS and becomes the bf16 B operand in
-//     registers right before the MFMA.  INT4: one 32-bit read of 8 nibbles, one shift
-//     and one AND-OR per bf16 pair (nibble q+8 in the low mantissa bits of bf16 128.0
-//     reads 136+q).  INT8: one 64-bit read of 8 bytes q+128, each converted exactly
-//     (integers below 256 are exact in bf16).  bf16: one 128-bit read, no conversion.
-//   * The offset the stored codes carry (136 * sum(x) for INT4, 128 * sum(x) for INT8)
-//     is taken out on the MFMA: the A operand times an all -136 (-128) B operand gives
-//     -136 * (row sum) in exactly the accumulator layout of the output tiles.  INT4
-//     scales each group's sum by its fp16 scale when the group (two k steps) completes;
-//     INT8 scales the whole sum by the row's fp32 scale after the split-K merge.
-//     Products are exact and accumulation is fp32.
+//     set by which global chunk each lane fetches: 16-byte chunk c of row r sits at a
+//     slot c ^ f(r) of the row (xsw, wslot), such that the 16 lanes that a 128-bit LDS read
+//     serves at once (rows 0-3 and 12-15 of one k block, rows 4-11 of the next) fall into
+//     distinct banks: no conflicts counted, against half of the LDS cycles before.
+//   * The k loop reads the operands of one 32-value slice while the MFMAs of the slice
+//     before run, also across the barrier between two steps, and converts the next
+//     slice's weights between those MFMAs (one set of A registers, refilled row by row).
+//     2048 x 28672 x 4096: bf16 574 -> 430 us (1.12 PFLOP/s), INT8 781 -> 460 us, INT4
+//     669 -> 505 us against the loop that read, converted and multiplied in turn.
+//   * Blocks are dealt to the XCDs in contiguous eighths of the tiles, so that weight and
+//     row tiles are shared in one L2 (bf16 as above: 453 instead of 566 us at 128 x 256).
+//   * The weight stays in its storage format in LDS.  INT4: signed nibble conversions
+//     (v_cvt_off_f32_i4 gives q / 16 exactly), two packed into a register.  INT8: signed
+//     byte conversions.  Both are exact in bf16.  Products are exact and accumulation is
+//     fp32.  bf16: one 128-bit read, no conversion.
+//   * INT4 group scales: the sums are kept in units of the running group's scale, so a
+//     new group costs one multiplication by old / new scale per sum and no second set of
+//     accumulators (which held the tile at 64 x 64 per wave); the last scale comes at the
+//     end.  The error against 64 bits is that of the bf16 outputs (0.0061 at 512 rows,
+//     before and now).
 //   * Rows past the M or N edge read row 0 and are never stored.
-//   * The INT4 k loop runs one group per iteration: the group's first MFMAs start from
-//     a zero accumulator, so closing a group is one fma per output and no clearing.
 //   * Split-K (tiles that would leave CUs idle): split s of a tile owns a contiguous
 //     range of whole groups (128 k values for INT8 and bf16).  Each split block stores
 //     its fp32 accumulators with device-scope stores, waits for them, and takes a ticket;
@@ -56,62 +60,108 @@ namespace {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((address_space(1))) void gvoid;
 typedef __attribute__((address_space(3))) void lvoid;
 
-constexpr int QBM = 128, QBK = 64;
+constexpr int QBK = 64;  // the k granule: a split's and a group's length are multiples of it
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 // Split-K partials move as 16-byte buffer loads and stores carrying the sc1 cache
 // policy (bit 4 of the builtins' aux operand on gfx950): the device-coherent accesses
 // the relaxed agent-scope atomics compile to, four words at a time.  The descriptor's
 // last dword is the raw-buffer format word (32-bit data, no swizzle); a wave's region
-// is 16 tiles x 64 lanes x 16 bytes.
+// is one 64 lanes x 16 bytes record per MFMA tile of the wave.
 constexpr int kCpolSc1 = 16;
 constexpr int kRawBufferFlags = 0x00020000;
-constexpr int kPartWaveBytes = 16 * 64 * 16;
-constexpr int XST = QBM * QBK * 2;  // 16 KB of X per stage
 
-// Bytes of one weight row per k step of 64, and the 16-byte chunks they make.
+// Bytes of 64 k values of one weight row.
 template <int WF> struct WRow;
 template <> struct WRow<AM_WF_INT4> { static constexpr int kBytes = 32; };
 template <> struct WRow<AM_WF_INT8> { static constexpr int kBytes = 64; };
 template <> struct WRow<AM_WF_BF16> { static constexpr int kBytes = 128; };
 
-// Block shapes: NWN waves along N (64 columns each) by 2 along M.
-//   NWN = 2: 256 threads, 128 x 128 tile, 3 stages (INT4 62 KB of LDS and INT8 72 KB:
-//            two blocks per CU; bf16 96 KB: one)
-//   NWN = 4: 512 threads, 128 x 256 tile, 4 stages (3 for bf16; INT4 100 KB, INT8
-//            128 KB, bf16 144 KB, one block per CU): half the X bytes per MFMA, which
-//            moves most of the traffic.
-template <int WF, int NWN>
-struct Shape {
+// Block shapes.  MW x NW waves, each MT x NT MFMA tiles of 16 x 16, a k step of BK
+// values, NST DMA stages, BPC resident blocks per CU to compile for.
+//   Quantized weights: one wave row (MW = 1), so that each weight is converted by one wave
+//   only.  LDS reads of X cost less than conversions (256 bytes against 16 weights' 28
+//   VALU operations per clock and CU): 2048 x 28672 x 4096 INT4 654 -> 546 us, INT8 535 ->
+//   476 us on the 128 x 256 tile.  bf16 weights need no conversion: two wave rows, which
+//   read the least from LDS.  The 256 x 256 tile keeps two rows in every format (one row
+//   of 16 x 2 tiles per wave does not fit the registers).
+//   INT4 takes 128 k values a step where LDS allows it (half the barriers and scale
+//   loads: 546 -> 505 us on the shape above).
+enum Tile { kT128 = 0, kT256 = 1, kT64 = 2, kT64W = 3, kT256x256 = 4 };
+template <int WF, int TILE> struct TileCfg;
+//   128 x 128, 256 threads (INT4 62 KB of LDS and INT8 72 KB: two blocks per CU; bf16
+//   96 KB: one)
+template <int WF> struct TileCfg<WF, kT128> {
+  static constexpr bool kB = WF == AM_WF_BF16;
+  static constexpr int MT = kB ? 4 : 8, NT = kB ? 4 : 2, MW = kB ? 2 : 1, NW = kB ? 2 : 4, BK = 64, NST = 3, BPC = 2;
+};
+//   128 x 256, 512 threads, one block per CU
+template <int WF> struct TileCfg<WF, kT256> {
+  static constexpr bool kB = WF == AM_WF_BF16;
+  static constexpr int MT = kB ? 4 : 8, NT = kB ? 4 : 2, MW = kB ? 2 : 1, NW = kB ? 4 : 8,
+                       BK = WF == AM_WF_INT4 ? 128 : 64, NST = WF == AM_WF_INT8 ? 4 : 3, BPC = 1;
+};
+//   64 x 64 (256 threads) and 64 x 128 (512 threads) for few rows, two blocks per CU
+template <int WF> struct TileCfg<WF, kT64> {
+  static constexpr bool kB = WF == AM_WF_BF16;
+  static constexpr int MT = kB ? 2 : 4, NT = kB ? 2 : 1, MW = kB ? 2 : 1, NW = kB ? 2 : 4,
+                       BK = WF == AM_WF_INT4 ? 128 : 64, NST = WF == AM_WF_INT4 ? 3 : (WF == AM_WF_INT8 ? 6 : 4), BPC = 2;
+};
+template <int WF> struct TileCfg<WF, kT64W> {
+  static constexpr bool kB = WF == AM_WF_BF16;
+  static constexpr int MT = kB ? 2 : 4, NT = kB ? 2 : 1, MW = kB ? 2 : 1, NW = kB ? 4 : 8,
+                       BK = WF == AM_WF_INT4 ? 128 : 64, NST = WF == AM_WF_INT4 ? 3 : (WF == AM_WF_INT8 ? 4 : 3), BPC = 2;
+};
+//   256 x 256, 512 threads, one block per CU: the fewest X and W bytes per MFMA
+template <int WF> struct TileCfg<WF, kT256x256> {
+  static constexpr int MT = 8, NT = 4, MW = 2, NW = 4, BK = 64, NST = WF == AM_WF_BF16 ? 2 : 3, BPC = 1;
+};
+template <int WF, int TILE>
+struct Shape : TileCfg<WF, TILE> {
+  using C = TileCfg<WF, TILE>;
   static constexpr bool kI4 = WF == AM_WF_INT4;
-  static constexpr int kWaves = 2 * NWN;
+  static constexpr int kWaves = C::MW * C::NW;
   static constexpr int kThreads = 64 * kWaves;
-  static constexpr int kBN = 64 * NWN;
-  static constexpr int kStages = NWN == 2 ? 3 : (WF == AM_WF_BF16 ? 3 : 4);
-  static constexpr int kRowB = WRow<WF>::kBytes;   // W row bytes per k step
+  static constexpr int kBM = 16 * C::MT * C::MW, kBN = 16 * C::NT * C::NW;
+  static constexpr int kXRow = C::BK * 2;                      // X row bytes per k step
+  static constexpr int kRowB = WRow<WF>::kBytes * C::BK / 64;  // W row bytes per k step
+  static constexpr int kXSt = kBM * kXRow;         // X bytes per stage
   static constexpr int kWSt = kBN * kRowB;         // W bytes per stage
-  static constexpr int kStg = XST + kWSt;
+  static constexpr int kStg = kXSt + kWSt;
   static constexpr int kScSlot = kBN * 4;          // INT4: one dword per weight row
-  static constexpr int kLds = kStages * kStg + (kI4 ? 4 * kScSlot : 0);
-  static constexpr int kXi = 16 / kWaves;          // X DMA instructions per wave per step
-  static constexpr int kWi = kWSt / 1024 / kWaves; // W DMA instructions per wave per step
+  static constexpr int kScSlots = 4;               // groups whose scales may be in LDS
+  static constexpr int kEpi = kBM * (kBN + 8) * 2;  // the epilogue's bf16 tile
+  static constexpr int kRing = C::NST * kStg + (kI4 ? kScSlots * kScSlot : 0);
+  static constexpr int kLds = kRing > kEpi ? kRing : kEpi;
+  static constexpr int kXi = kXSt / 1024 / kWaves;  // X DMA instructions per wave per step
+  static constexpr int kWi = kWSt / 1024 / kWaves;  // W DMA instructions per wave per step
   static constexpr int kLoads = kXi + kWi + (kI4 ? 1 : 0);  // + the INT4 scale dword
+  static constexpr int kTiles = C::MT * C::NT;              // MFMA tiles per wave
+  static constexpr int kPartWave = kTiles * 64 * 4;         // fp32 partials of a wave
+  static_assert(C::BK % 64 == 0, "the loop's operand sets alternate over an even number of slices");
+  static_assert(kXi >= 1 && kXi * kWaves * 1024 == kXSt, "X stage must be whole DMA instructions per wave");
   static_assert(kWi >= 1 && kWi * kWaves * 1024 == kWSt, "W stage must be whole DMA instructions per wave");
+  static_assert(C::NST <= 6 && kLoads * (C::NST - 1) < 64, "the memory counter must hold the steps in flight");
+  static_assert(!kI4 || C::NST <= kScSlots || C::BK == 64, "a group's scales must outlive the steps in flight");
 };
 
-// Slot of 16-byte chunk c of weight row n within the row's k-step bytes.
-template <int WF>
+// Slot of 16-byte chunk c of weight row n within the row's k-step bytes (RB of them).
+template <int RB>
 __device__ __forceinline__ int wslot(int n, int c) {
-  if constexpr (WF == AM_WF_INT4) return c ^ ((n >> 3) & 1);
-  else if constexpr (WF == AM_WF_INT8) return c ^ ((n >> 2) & 3);
-  else return c ^ ((n & 7) ^ ((n >> 3) & 1));
+  if constexpr (RB == 32) return c ^ ((n >> 3) & 1);
+  else if constexpr (RB == 64) return c ^ ((n >> 2) & 3);
+  else return c ^ ((n >> 1) & 7);
 }
 
-// X row r's 16-byte chunk c sits at slot c ^ xsw(r) of the row: 8 consecutive rows, and
-// 16 rows taken as two parity classes, land in distinct LDS banks.
-__device__ __forceinline__ int xsw(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+// X row r's 16-byte chunk c sits at slot c ^ xsw(r) of the row: with 128-byte rows 8
+// consecutive rows, and 16 rows taken as two parity classes, land in distinct LDS
+// banks; with 256-byte rows all 16 do.
+template <int BK>
+__device__ __forceinline__ int xsw(int r) {
+  if constexpr (BK == 128) return r & 15;
+  else return (r >> 1) & 7;
+}
 
 enum I4Epi { kI4Store = 0, kI4Residual = 1, kI4Split = 2, kI4SiluMul = 3, kI4QkvRope = 4 };
 
@@ -142,258 +192,366 @@ struct I4Args {
   int32_t* err;               // optional: set when a row's position is outside [0, cap)
 };
 
-// 8 bytes q+128 -> 8 exact bf16 values 0..255, in byte order
+// 8 bytes q+128 -> 8 bf16 values q (exact), in byte order: signed byte conversions, and
+// the top halves of the fp32 bits of small integers are their bf16 encodings.
 __device__ __forceinline__ bf16x8_t bytes8(uint2 v) {
-  const uint32_t w[2] = {v.x, v.y};
+  const uint32_t w[2] = {v.x ^ 0x80808080u, v.y ^ 0x80808080u};
   uint32_t d[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t word = w[i >> 1];
-    const int sh = 16 * (i & 1);
-    const float lo = static_cast<float>((word >> sh) & 0xFFu), hi = static_cast<float>((word >> (sh + 8)) & 0xFFu);
-    const bf16x2_t h = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-    d[i] = __builtin_bit_cast(uint32_t, h);
+    const uint32_t word = w[i >> 1] >> (16 * (i & 1));
+    const float lo = static_cast<float>(static_cast<int8_t>(word)), hi = static_cast<float>(static_cast<int8_t>(word >> 8));
+    d[i] = __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
   }
   return __builtin_bit_cast(bf16x8_t, make_uint4(d[0], d[1], d[2], d[3]));
 }
 
-__device__ __forceinline__ bf16x8_t unpack8(uint32_t word, uint32_t mask, uint32_t magic) {
-  uint32_t d[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) d[i] = ((word >> (4 * i)) & mask) | magic;
-  return __builtin_bit_cast(bf16x8_t, make_uint4(d[0], d[1], d[2], d[3]));
+// signed 4-bit value of the low nibble of byte B of v, over 16 (v_cvt_off_f32_i4)
+template <int B>
+__device__ __forceinline__ uint32_t nibble16(uint32_t v) {
+  uint32_t d;
+  if constexpr (B == 0) asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(d) : "v"(v));
+  else if constexpr (B == 1) asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(d) : "v"(v));
+  else if constexpr (B == 2) asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(d) : "v"(v));
+  else asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(d) : "v"(v));
+  return d;
 }
 
-__device__ __forceinline__ void dma16(const void* g, uint8_t* l) {
-  __builtin_amdgcn_global_load_lds((const gvoid*)(g), (lvoid*)(l), 16, 0, 0);
-}
-__device__ __forceinline__ void dma4(const void* g, uint8_t* l) {
-  __builtin_amdgcn_global_load_lds((const gvoid*)(g), (lvoid*)(l), 4, 0, 0);
+// 8 nibbles q+8 in device tile order -> 8 bf16 values q / 16 (exact) in k order: the
+// nibbles of k 0, 4, 1, 5 are the low halves of bytes 0..3, those of k 2, 6, 3, 7 the
+// high halves.
+__device__ __forceinline__ bf16x8_t unpack8(uint32_t word) {
+  const uint32_t lo = word ^ 0x88888888u, hi = lo >> 4;
+  const uint32_t d0 = __builtin_amdgcn_perm(nibble16<2>(lo), nibble16<0>(lo), 0x07060302u);
+  const uint32_t d1 = __builtin_amdgcn_perm(nibble16<2>(hi), nibble16<0>(hi), 0x07060302u);
+  const uint32_t d2 = __builtin_amdgcn_perm(nibble16<3>(lo), nibble16<1>(lo), 0x07060302u);
+  const uint32_t d3 = __builtin_amdgcn_perm(nibble16<3>(hi), nibble16<1>(hi), 0x07060302u);
+  return __builtin_bit_cast(bf16x8_t, make_uint4(d0, d1, d2, d3));
 }
 
-// Weight row of local tile row r.
+// Global -> LDS DMA of 16 (4) bytes per lane: lane L's bytes at base + off land at LDS
+// byte lds + 16 (4) L.  Written as asm because the compiler counts the builtin's LDS
+// write against every later LDS read and may wait for all DMA in flight before each one
+// (vmcnt(0) in the k loop); the loop waits for exactly the steps it needs.  No register
+// is written, and the address registers are read at issue.
+__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void dma4(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+
+// Weight row of local tile row r.  SiLU-Mul: the first half of a tile's rows are gate
+// features, the second half the up rows of the same features.  RoPE with heads wider
+// than the tile: the first half of the rows lie in the first half of a head, the second
+// half are their rotation partners d/2 later.
 template <int EPI, int BN>
 __device__ __forceinline__ int32_t wrow(const I4Args& p, int32_t tn, int32_t r) {
   if constexpr (EPI == kI4SiluMul) return r < BN / 2 ? tn * (BN / 2) + r : p.ffn + tn * (BN / 2) + (r - BN / 2);
+  if constexpr (EPI == kI4QkvRope && BN < 128) {
+    if (p.hd > BN) {
+      const int32_t per = p.hd / BN, head = tn / per, base = head * p.hd + (tn - head * per) * (BN / 2);
+      return r < BN / 2 ? base + r : base + (p.hd >> 1) + (r - BN / 2);
+    }
+  }
   const int32_t g = tn * BN + r;
   return g < p.N ? g : 0;
 }
 
-// Wait until at most AHEAD steps of this wave's DMA are in flight, then a plain
+// Wait for this wave's LDS reads, in a form the compiler's own wait insertion sees (an asm
+// wait it does not): it then knows that nothing is pending.
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
+
+// Wait until at most AHEAD (<= MAX) steps of this wave's DMA are in flight, then a plain
 // s_barrier, as one asm statement (no memory access moves across it; a fenced barrier
 // would also wait for the younger steps' DMA).
-template <int LOADS>
+template <int LOADS, int MAX>
 __device__ __forceinline__ void wait_barrier(int ahead) {
-  if (ahead >= 2)
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * LOADS) : "memory");
-  else if (ahead == 1)
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LOADS) : "memory");
-  else
+  if constexpr (MAX > 0) {
+    if (ahead >= MAX)
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(MAX * LOADS) : "memory");
+    else
+      wait_barrier<LOADS, MAX - 1>(ahead);
+  } else {
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  }
 }
 
-template <int WF, int EPI, int NWN>
-__global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void gemm_mfma_kernel(I4Args p) {
-  using S = Shape<WF, NWN>;
-  constexpr int BN = S::kBN, NST = S::kStages, STG = S::kStg;
+template <int WF, int EPI, int TILE>
+__global__ __launch_bounds__((Shape<WF, TILE>::kThreads), (Shape<WF, TILE>::BPC)) void gemm_mfma_kernel(I4Args p) {
+  using S = Shape<WF, TILE>;
+  constexpr int BM = S::kBM, BN = S::kBN, NST = S::NST, STG = S::kStg, MT = S::MT, NT = S::NT, NW = S::NW;
+  constexpr int BK = S::BK, KK = BK / 32, XST = S::kXSt, XROW = S::kXRow, RB = S::kRowB;
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / NWN, wn = wave % NWN;
+  const int wm = wave / NW, wn = wave % NW;
+  // arguments of the epilogue in registers now (see the loop)
+  uint16_t* out0 = p.out0;
+  const uint16_t* residual = p.residual;
+  asm volatile("" : "+s"(out0), "+s"(residual));
 
   // tile mapping: bands of 8 M-tiles, N fastest inside a band
-  const int32_t tiles_m = (p.M + QBM - 1) / QBM;
+  const int32_t tiles_m = (p.M + BM - 1) / BM;
   const int32_t tiles_n = EPI == kI4SiluMul ? p.ffn / (BN / 2) : (p.N + BN - 1) / BN;
   const int32_t tiles = tiles_m * tiles_n;
-  const int32_t split = blockIdx.x / tiles;
-  const int32_t bid = blockIdx.x - split * tiles;
+  // Block b runs on XCD b mod 8, each with an L2 of its own: XCD x takes the x-th
+  // contiguous eighth of the launch's tiles, so the M tiles that share a weight tile (and
+  // the N tiles that share rows of X) meet in one L2.
+  const int32_t xq = gridDim.x >> 3, xr = gridDim.x & 7, xcd = blockIdx.x & 7;
+  const int32_t lin = xcd * xq + min(xcd, xr) + static_cast<int32_t>(blockIdx.x >> 3);
+  const int32_t bid = lin / p.splits;
+  const int32_t split = lin - bid * p.splits;
   const int32_t per_band = 8 * tiles_n;
   const int32_t b0 = bid / per_band, rem = bid - b0 * per_band;
   const int32_t bands_m = min(tiles_m - b0 * 8, 8);
   const int32_t tm = b0 * 8 + rem % bands_m, tn = rem / bands_m;
-  const int32_t m0 = tm * QBM;
+  const int32_t m0 = tm * BM;
 
   const int32_t ng = p.K / p.group;
-  const int32_t spg = p.group / QBK;  // k steps per group
+  const int32_t spg = p.group / BK;  // k steps per group
   // this split's groups [g0, g1) = k steps [k0, k0 + nk)
   const int32_t g0 = split * ng / p.splits, g1 = (split + 1) * ng / p.splits;
   const int32_t k0 = g0 * spg, nk = (g1 - g0) * spg;
 
   // ---- DMA sources of this lane ----
-  // X: wave w moves rows [8 kXi w, 8 kXi (w + 1)), 8 rows per instruction
-  const uint8_t* xsrc[S::kXi];
+  // X: an instruction moves 1 KB, 1024 / XROW rows
+  constexpr int XPI = 1024 / XROW, XCH = XROW / 16;
+  uint32_t xsrc[S::kXi];  // byte offsets (M * K and N rows stay below 2^31 elements and bytes)
 #pragma unroll
   for (int i = 0; i < S::kXi; ++i) {
-    const int r = (wave * S::kXi + i) * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ xsw(r);
+    const int r = (wave * S::kXi + i) * XPI + lane / XCH;
+    const int c = (lane % XCH) ^ xsw<BK>(r);
     const int32_t gr = m0 + r < p.M ? m0 + r : 0;
-    xsrc[i] = reinterpret_cast<const uint8_t*>(p.x) + (static_cast<int64_t>(gr) * p.K + 8 * c) * 2;
+    xsrc[i] = static_cast<uint32_t>((static_cast<int64_t>(gr) * p.K + 8 * c) * 2);
   }
-  // INT8: the fp32 scales of this lane's four output columns, loaded ahead of every DMA
-  float rs[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+  // INT8: the fp32 scales of this lane's output columns, loaded ahead of every DMA
+  float rs[NT];
   if constexpr (WF == AM_WF_INT8) {
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-      rs[nt] = static_cast<const float*>(p.s)[wrow<EPI, BN>(p, tn, wn * 64 + nt * 16 + (lane & 15))];
+    for (int nt = 0; nt < NT; ++nt)
+      rs[nt] = static_cast<const float*>(p.s)[wrow<EPI, BN>(p, tn, (wn * NT + nt) * 16 + (lane & 15))];
   }
   // W: instruction i of wave w fills 1 KB of the stage's W rows; lane L's 16 bytes land
   // at row (1024 (w kWi + i) + 16 L) / kRowB, slot ((16 L) mod kRowB) / 16, so it fetches
   // the chunk whose slot that is (the slot map is an XOR, its own inverse)
-  const int64_t wrow_bytes = static_cast<int64_t>(p.K) / QBK * S::kRowB;
-  const uint8_t* wsrc[S::kWi];
+  const int64_t wrow_bytes = static_cast<int64_t>(p.K) / BK * RB;
+  uint32_t wsrc[S::kWi];
 #pragma unroll
   for (int i = 0; i < S::kWi; ++i) {
     const int o = (wave * S::kWi + i) * 1024 + 16 * lane;
-    const int r = o / S::kRowB, slot = (o % S::kRowB) / 16;
-    wsrc[i] = p.w + static_cast<int64_t>(wrow<EPI, BN>(p, tn, r)) * wrow_bytes + 16 * wslot<WF>(r, slot);
+    const int r = o / RB, slot = (o % RB) / 16;
+    wsrc[i] = static_cast<uint32_t>(static_cast<int64_t>(wrow<EPI, BN>(p, tn, r)) * wrow_bytes + 16 * wslot<RB>(r, slot));
   }
-  // INT4 scales: lane -> weight row (wave % NWN) * 64 + lane (waves past NWN repeat the
-  // same rows); the dword holding its fp16
-  const int sr = (wave % NWN) * 64 + lane;
+  // INT4 scales: lane -> weight row 64 (wave % (BN / 64)) + lane (the other waves repeat
+  // the same rows); the dword holding its fp16
+  const int sr = (wave % (BN / 64)) * 64 + lane;
   const int64_t sbase = S::kI4 ? static_cast<int64_t>(wrow<EPI, BN>(p, tn, sr)) * ng : 0;
 
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lvoid*)(lds)));
   auto issue = [&](int32_t j) {  // local step j = k step k0 + j
     const int32_t ks = k0 + j;
-    uint8_t* st = lds + (j % NST) * STG;
+    const uint32_t st = lds0 + (j % NST) * STG;
+    const uint8_t* xb = reinterpret_cast<const uint8_t*>(p.x) + static_cast<int64_t>(ks) * XROW;
+    const uint8_t* wb = p.w + static_cast<int64_t>(ks) * RB;
 #pragma unroll
-    for (int i = 0; i < S::kXi; ++i) dma16(xsrc[i] + ks * (QBK * 2), st + (wave * S::kXi + i) * 1024);
+    for (int i = 0; i < S::kXi; ++i) dma16(xb, xsrc[i], st + (wave * S::kXi + i) * 1024);
 #pragma unroll
-    for (int i = 0; i < S::kWi; ++i) dma16(wsrc[i] + ks * S::kRowB, st + XST + (wave * S::kWi + i) * 1024);
+    for (int i = 0; i < S::kWi; ++i) dma16(wb, wsrc[i], st + XST + (wave * S::kWi + i) * 1024);
     if constexpr (S::kI4) {
       const int32_t g = ks / spg;
       const int64_t se = sbase + g;  // fp16 element; its dword, aligned down
-      dma4(reinterpret_cast<const uint8_t*>(p.s) + ((se * 2) & ~int64_t{3}),
-           lds + NST * STG + (g & 3) * S::kScSlot + (wave % NWN) * 256);
+      dma4(p.s, static_cast<uint32_t>((se * 2) & ~int64_t{3}),
+           lds0 + NST * STG + (g & (S::kScSlots - 1)) * S::kScSlot + (wave % (BN / 64)) * 256);
     }
   };
 
-  f32x4_t acc[4][4], part[4][4], corr[4];
+  const f32x4_t zero4 = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t acc[MT][NT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    corr[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      part[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-  }
-  uint32_t mask = 0x000F000Fu, magic = 0x43004300u;
-  asm volatile("" : "+v"(mask), "+v"(magic));
-  // the code offset times -1 (INT4 -136, INT8 -128) as an all-equal B operand
-  constexpr uint32_t kNeg = S::kI4 ? 0xC308C308u : 0xC300C300u;
-  constexpr bool kOff = WF != AM_WF_BF16;
-  const bf16x8_t bneg = __builtin_bit_cast(bf16x8_t, make_uint4(kNeg, kNeg, kNeg, kNeg));
+    for (int j = 0; j < NT; ++j) acc[i][j] = zero4;
 
-  // LDS read offsets of this lane (within a stage)
-  int aoff[4][2], boff[4][2];
+  // LDS read offsets of this lane (within a stage).  Lane group kb takes the 8 k values
+  // 32 kk + 8 kb + ... of MFMA kk.
+  const int kb = lane >> 4;
+  int aoff[MT][KK], boff[NT][KK];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int r = wm * 64 + mt * 16 + (lane & 15);
+  for (int mt = 0; mt < MT; ++mt) {
+    const int r = (wm * MT + mt) * 16 + (lane & 15);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) aoff[mt][kk] = r * 128 + 16 * ((kk * 4 + (lane >> 4)) ^ xsw(r));
+    for (int kk = 0; kk < KK; ++kk) aoff[mt][kk] = r * XROW + 16 * ((kk * 4 + kb) ^ xsw<BK>(r));
   }
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const int n = wn * 64 + nt * 16 + (lane & 15);
-    const int kb = lane >> 4;  // 8-value k block of this lane's B operand
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = (wn * NT + nt) * 16 + (lane & 15);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
+    for (int kk = 0; kk < KK; ++kk) {
       if constexpr (WF == AM_WF_INT4)
-        boff[nt][kk] = XST + n * 32 + 16 * wslot<WF>(n, kk) + 4 * kb;
+        boff[nt][kk] = XST + n * RB + 16 * wslot<RB>(n, kk) + 4 * kb;
       else if constexpr (WF == AM_WF_INT8)
-        boff[nt][kk] = XST + n * 64 + 16 * wslot<WF>(n, 2 * kk + (kb >> 1)) + 8 * (kb & 1);
+        boff[nt][kk] = XST + n * RB + 16 * wslot<RB>(n, 2 * kk + (kb >> 1)) + 8 * (kb & 1);
       else
-        boff[nt][kk] = XST + n * 128 + 16 * wslot<WF>(n, 4 * kk + kb);
+        boff[nt][kk] = XST + n * RB + 16 * wslot<RB>(n, 4 * kk + kb);
     }
   }
   // scale of this lane's column of tile nt in group g: the half of the slot dword that
   // holds element (row * ng + g)
-  int soff[4], shalf_base[4];
+  // (tiles, features and heads start at even rows, so a row's parity is its lane's)
+  const int soff = NST * STG + (wn * NT * 16 + (lane & 15)) * 4;
+  const int shalf = lane & ng & 1;
+
+  // Operands of one MFMA k slice: A as read, B in storage format and as bf16 (two slices)
+  using RawB = std::conditional_t<WF == AM_WF_INT4, uint32_t, std::conditional_t<WF == AM_WF_INT8, uint2, uint4>>;
+  uint4 oa[MT];
+  RawB ob[NT];
+  bf16x8_t bfr[2][NT];
+  uint32_t sraw[NT];       // INT4: the group's scale dwords
+  float sc[NT];            // INT4: the scale the sums are in units of
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const int n = wn * 64 + nt * 16 + (lane & 15);
-    soff[nt] = NST * STG + n * 4;
-    shalf_base[nt] = S::kI4 ? static_cast<int>(static_cast<int64_t>(wrow<EPI, BN>(p, tn, n)) * ng & 1) : 0;
+  for (int nt = 0; nt < NT; ++nt) {
+    sc[nt] = 1.0f;
+    sraw[nt] = 0u;
   }
-
-  // prologue: steps 0 .. NST-2 in flight
+  auto fetch_a = [&](const uint8_t* st, int kk, int mt) { oa[mt] = *reinterpret_cast<const uint4*>(st + aoff[mt][kk]); };
+  auto fetch_b = [&](const uint8_t* st, int kk) {
 #pragma unroll
-  for (int i = 0; i < NST - 1; ++i)
-    if (i < nk) issue(i);
-
-  const f32x4_t zero4 = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  // one k step: FIRST starts the group's partial sums from zero
-  auto step = [&](int32_t j, auto first_tag) {
-    constexpr bool FIRST = decltype(first_tag)::value;
-    // this wave's DMA for step j has landed (younger steps may still be in flight);
-    // after the barrier every wave's has, and step j-1 is no longer read
-    static_assert(NST <= 4, "wait_barrier keeps at most two younger steps in flight");
-    wait_barrier<S::kLoads>(min(nk - 1 - j, NST - 2));
-    if (j + NST - 1 < nk) issue(j + NST - 1);
-    const uint8_t* st = lds + (j % NST) * STG;
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      bf16x8_t af[4], bfr[4];
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) af[mt] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(st + aoff[mt][kk]));
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        if constexpr (WF == AM_WF_INT4)
-          bfr[nt] = unpack8(*reinterpret_cast<const uint32_t*>(st + boff[nt][kk]), mask, magic);
-        else if constexpr (WF == AM_WF_INT8)
-          bfr[nt] = bytes8(*reinterpret_cast<const uint2*>(st + boff[nt][kk]));
-        else
-          bfr[nt] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(st + boff[nt][kk]));
-      }
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-        if constexpr (kOff)
-          corr[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[mt], bneg, (FIRST && kk == 0) ? zero4 : corr[mt], 0, 0, 0);
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
-          part[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[mt], bfr[nt], (FIRST && kk == 0) ? zero4 : part[mt][nt],
-                                                                 0, 0, 0);
-      }
+    for (int nt = 0; nt < NT; ++nt) {
+      if constexpr (WF == AM_WF_BF16)
+        bfr[kk & 1][nt] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const RawB*>(st + boff[nt][kk]));
+      else
+        ob[nt] = *reinterpret_cast<const RawB*>(st + boff[nt][kk]);
     }
   };
+  auto convert = [&](int nt, int kk) {
+    if constexpr (WF == AM_WF_INT4) bfr[kk & 1][nt] = unpack8(ob[nt]);
+    else if constexpr (WF == AM_WF_INT8) bfr[kk & 1][nt] = bytes8(ob[nt]);
+  };
+  auto fetch_scales = [&](int32_t g) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+      sraw[nt] = *reinterpret_cast<const uint32_t*>(lds + soff + nt * 64 + (g & (S::kScSlots - 1)) * S::kScSlot);
+  };
+  // A group begins: the sums so far change to its unit.  A zero scale counts as 2^-60:
+  // the codes the quantizer stores with it are 0, and others vanish beside any sum.
+  auto open_group = [&](int32_t g, float (&ratio)[NT]) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const uint32_t bits = ((shalf + g) & 1) ? (sraw[nt] >> 16) : (sraw[nt] & 0xFFFFu);
+      float s = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(bits)));
+      if (s == 0.0f) s = 0x1p-60f;
+      // sc / s: reciprocal and one correction (not where that meets an infinity)
+      const float inv = __builtin_amdgcn_rcpf(s);
+      float q = sc[nt] * inv;
+      const float e = __builtin_fmaf(-q, s, sc[nt]);
+      if (e == e) q = __builtin_fmaf(e, inv, q);
+      ratio[nt] = s == sc[nt] ? 1.0f : q;
+      sc[nt] = s;
+    }
+  };
+  // MFMAs of slice kk; RESCALE: the first slice of an INT4 group.  As soon as a row of
+  // tiles is issued its A registers take the operand of the next slice (kn of step sn),
+  // and in the second half of the rows the next slice's weights are converted: LDS reads
+  // and conversions run behind the MFMAs, kept there by the barriers to reordering.
+  auto slice = [&](int kk, const uint8_t* sn, int kn, auto rescale, const float (&ratio)[NT]) {
+    constexpr bool RESCALE = decltype(rescale)::value;
+    fetch_b(sn, kn);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const bf16x8_t af = __builtin_bit_cast(bf16x8_t, oa[mt]);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        if constexpr (RESCALE) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[mt][nt][r] *= ratio[nt];
+        }
+        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr[kk & 1][nt], acc[mt][nt], 0, 0, 0);
+      }
+      fetch_a(sn, kn, mt);
+      constexpr int H = MT / 2;
+      if constexpr (WF != AM_WF_BF16) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          if (H + nt * H / NT == mt) convert(nt, kk + 1);
+      }
+      if constexpr (MT > 4 || WF != AM_WF_BF16) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // prologue: steps 0 .. NST-1 in flight, then the first slice's operands
+#pragma unroll
+  for (int i = 0; i < NST; ++i)
+    if (i < nk) issue(i);
+  wait_barrier<S::kLoads, NST - 1>(nk - 1);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) fetch_a(lds, 0, mt);
+  fetch_b(lds, 0);
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) convert(nt, 0);
+  if constexpr (S::kI4) fetch_scales(g0);
+  // no scalar load may be pending when the loop begins, or the compiler waits for all LDS
+  // reads at each use in it
+  __builtin_amdgcn_sched_barrier(0);
+  wait_lds();
+  __builtin_amdgcn_sched_barrier(0);
+
+  // One slice of operands is read from LDS while the MFMAs of the slice before run.  The
+  // last slice of a step runs after the barrier that ends the step: every wave has then
+  // read all of the step, so its slot takes the DMA of step j + NST, and the next
+  // step's first operands are read behind those MFMAs (after the last step: bytes of an
+  // older one, never used).
+  auto step = [&](int32_t j, int32_t next_group, auto first, const float (&ratio)[NT]) {
+    const uint8_t* st = lds + (j % NST) * STG;
+    const uint8_t* sn = lds + ((j + 1) % NST) * STG;
+    slice(0, st, 1, first, ratio);
+#pragma unroll
+    for (int kk = 1; kk + 1 < KK; ++kk) slice(kk, st, kk + 1, std::false_type{}, ratio);
+    if (j + 1 < nk) {
+      wait_lds();
+      wait_barrier<S::kLoads, NST - 2>(nk - 2 - j);
+      if (j + NST < nk) issue(j + NST);
+      if (S::kI4 && next_group >= 0) fetch_scales(next_group);
+    }
+    slice(KK - 1, sn, 0, std::false_type{}, ratio);
+  };
+  float ratio[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) ratio[nt] = 1.0f;
   int32_t j = 0;
   if constexpr (S::kI4) {
     for (int32_t g = g0; g < g1; ++g) {
-      step(j++, std::true_type{});
-      for (int32_t t = 1; t < spg; ++t) step(j++, std::false_type{});
-      // the group closes: scale and fold into acc
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const uint32_t sw = *reinterpret_cast<const uint32_t*>(lds + soff[nt] + (g & 3) * S::kScSlot);
-        const uint32_t bits = ((shalf_base[nt] + g) & 1) ? (sw >> 16) : (sw & 0xFFFFu);
-        const float sc = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(bits)));
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[mt][nt][r] = fmaf(sc, part[mt][nt][r] + corr[mt][r], acc[mt][nt][r]);
-      }
+      open_group(g, ratio);
+      step(j, spg == 1 ? g + 1 : -1, std::true_type{}, ratio);
+      ++j;
+      for (int32_t t = 1; t < spg; ++t, ++j) step(j, t + 1 == spg ? g + 1 : -1, std::false_type{}, ratio);
     }
   } else {
-    // one running sum over the split's k range (the row scale comes after the merge)
-    step(j++, std::true_type{});
-    while (j < nk) step(j++, std::false_type{});
+    for (; j < nk; ++j) step(j, -1, std::false_type{}, ratio);
+  }
+  if constexpr (S::kI4) {
+    // out of the last group's unit; the operands were q / 16
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
+      for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[mt][nt][r] = kOff ? part[mt][nt][r] + corr[mt][r] : part[mt][nt][r];
+        for (int r = 0; r < 4; ++r) acc[mt][nt][r] *= 16.0f * sc[nt];
   }
 
   if (p.splits > 1) {
     // partial of this split: device-scope (sc1) 16-byte buffer stores of the wave's
-    // 16 KB region, acknowledged before the ticket
-    float* mine = p.part + ((static_cast<int64_t>(bid) * p.splits + split) * S::kWaves + wave) * (16 * 64 * 4);
-    const __amdgpu_buffer_rsrc_t rmine = __builtin_amdgcn_make_buffer_rsrc(mine, 0, kPartWaveBytes, kRawBufferFlags);
+    // region, acknowledged before the ticket
+    constexpr int kTiles = S::kTiles, kWaveBytes = S::kPartWave * 4;
+    auto region = [&](int32_t sp) {
+      float* at = p.part + ((static_cast<int64_t>(bid) * p.splits + sp) * S::kWaves + wave) * S::kPartWave;
+      return __builtin_amdgcn_make_buffer_rsrc(at, 0, kWaveBytes, kRawBufferFlags);
+    };
+    const __amdgpu_buffer_rsrc_t rmine = region(split);
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i / 4][i % 4]), rmine, (i * 64 + lane) * 16, 0,
+    for (int i = 0; i < kTiles; ++i)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i / NT][i % NT]), rmine, (i * 64 + lane) * 16, 0,
                                              kCpolSc1);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -403,34 +561,33 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
              static_cast<unsigned>(p.splits - 1);
     __syncthreads();
     if (!last) return;
-    // the tile's sum in split order
-    f32x4_t sum[16];
+    // the tile's sum in split order, one row of MFMA tiles at a time (this split's own
+    // partial is read back too: its registers are free for the loads in flight)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) sum[i] = zero4;
-    for (int sp = 0; sp < p.splits; ++sp) {
-      if (sp == split) {
+    for (int mt = 0; mt < MT; ++mt) {
+      f32x4_t sum[NT];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sum[i] += acc[i / 4][i % 4];
-        continue;
+      for (int nt = 0; nt < NT; ++nt) sum[nt] = zero4;
+#pragma unroll 2
+      for (int sp = 0; sp < p.splits; ++sp) {
+        const __amdgpu_buffer_rsrc_t rsrc = region(sp);
+        u32x4_t v[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          v[nt] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, ((mt * NT + nt) * 64 + lane) * 16, 0, kCpolSc1);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) sum[nt] += __builtin_bit_cast(f32x4_t, v[nt]);
       }
-      const float* src = p.part + ((static_cast<int64_t>(bid) * p.splits + sp) * S::kWaves + wave) * (16 * 64 * 4);
-      const __amdgpu_buffer_rsrc_t rsrc =
-          __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, kPartWaveBytes, kRawBufferFlags);
-      u32x4_t v[16];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (i * 64 + lane) * 16, 0, kCpolSc1);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sum[i] += __builtin_bit_cast(f32x4_t, v[i]);
+      for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = sum[nt];
     }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i / 4][i % 4] = sum[i];
     if (tid == 0) __hip_atomic_store(&p.tickets[bid], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if constexpr (WF == AM_WF_INT8) {
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
+      for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[mt][nt][r] *= rs[nt];
   }
@@ -440,12 +597,12 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
   uint16_t* T = reinterpret_cast<uint16_t*>(lds);
   __syncthreads();  // every wave is done with the ring
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        T[(wm * 64 + mt * 16 + 4 * (lane >> 4) + r) * TS + wn * 64 + nt * 16 + (lane & 15)] =
+        T[((wm * MT + mt) * 16 + 4 * (lane >> 4) + r) * TS + (wn * NT + nt) * 16 + (lane & 15)] =
             f32_to_bf16_bits(acc[mt][nt][r]);
   __syncthreads();
 
@@ -454,18 +611,23 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
     // columns d/2 later (the RoPE partners), from the rounded tile.  q and k pairs are
     // rotated in fp32 from the bf16 values and rounded once (the RoPE node); k and v
     // go straight to the cache rows of their positions (the KVCacheUpdate node).
-    const int32_t d = p.hd, half = d >> 1, hpt = d >> 4;  // chunk pairs per head
+    const int32_t d = p.hd, half = d >> 1;
+    // tile columns of a head or of a piece of one (wrow): the partner of a first-half
+    // column lies pd / 2 columns later
+    const int32_t pd = min(d, BN), ph = pd >> 1, hpt = pd >> 4;  // hpt: chunk pairs per pd columns
+    const int32_t per = d / pd;                                  // pieces per head
     const int64_t start = *p.start;
-    constexpr int PPR = BN / 16;  // chunk pairs per tile row (BN is a multiple of d)
-    for (int c = tid; c < QBM * PPR; c += S::kThreads) {
+    constexpr int PPR = BN / 16;  // chunk pairs per tile row (BN is a multiple of pd)
+    for (int c = tid; c < BM * PPR; c += S::kThreads) {
       const int row = c / PPR, pr = c % PPR;
       const int32_t gm = m0 + row;
-      const int i0 = (pr % hpt) * 8;              // offset of the chunk inside its head
-      const int col = (pr / hpt) * d + i0;        // tile column of the first-half chunk
-      const int32_t gn = tn * BN + col;
+      const int col = (pr / hpt) * pd + (pr % hpt) * 8;  // tile column of the first-half chunk
+      const int32_t piece = tn % per;                    // 0 unless the head is wider than the tile
+      const int i0 = piece * ph + (pr % hpt) * 8;        // offset of the chunk inside its head
+      const int32_t gn = per > 1 ? (tn / per) * d + i0 : tn * BN + col;
       if (gm >= p.M || gn >= p.N) continue;
       const uint4 a1 = *reinterpret_cast<const uint4*>(T + row * TS + col);
-      const uint4 a2 = *reinterpret_cast<const uint4*>(T + row * TS + col + half);
+      const uint4 a2 = *reinterpret_cast<const uint4*>(T + row * TS + col + ph);
       const int64_t pos = start + gm;
       const bool ok = pos >= 0 && pos < p.cap;
       uint4 o1 = a1, o2 = a2;
@@ -498,7 +660,7 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
       }
       if (!ok && p.err != nullptr) *p.err = 1;
       if (gn < p.c1) {
-        uint16_t* dst = p.out0 + static_cast<int64_t>(gm) * p.c1 + gn;
+        uint16_t* dst = out0 + static_cast<int64_t>(gm) * p.c1 + gn;
         *reinterpret_cast<uint4*>(dst) = o1;
         *reinterpret_cast<uint4*>(dst + half) = o2;
       } else if (ok) {
@@ -517,7 +679,7 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
 
   if constexpr (EPI == kI4SiluMul) {
     constexpr int CPR = BN / 16;  // 16-byte output chunks per row (BN/2 features)
-    constexpr int IT = QBM * CPR / S::kThreads;
+    constexpr int IT = BM * CPR / S::kThreads;
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       const int c = tid + S::kThreads * i, row = c / CPR, cc = c % CPR;
@@ -525,7 +687,7 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
       if (gm >= p.M) continue;
       const uint16_t* gt = T + row * TS + cc * 8;
       const uint16_t* ut = gt + BN / 2;
-      uint16_t* o = p.out0 + static_cast<int64_t>(gm) * p.ffn + tn * (BN / 2) + cc * 8;
+      uint16_t* o = out0 + static_cast<int64_t>(gm) * p.ffn + tn * (BN / 2) + cc * 8;
       if (p.vec) {
         const uint4 gv = *reinterpret_cast<const uint4*>(gt), uv = *reinterpret_cast<const uint4*>(ut);
         const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
@@ -546,7 +708,7 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
   }
 
   constexpr int CPR = BN / 8;  // 16-byte chunks per tile row
-  constexpr int IT = QBM * CPR / S::kThreads;
+  constexpr int IT = BM * CPR / S::kThreads;
   // residual chunks first, all loads in flight (each thread reads only the chunks it
   // writes, so an aliased residual is read before it is overwritten)
   uint4 rres[EPI == kI4Residual ? IT : 1];
@@ -557,7 +719,7 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
         const int c = tid + S::kThreads * i, row = c / CPR, cc = c % CPR;
         const int32_t gm = m0 + row, gn = tn * BN + cc * 8;
         const int64_t idx = (gm < p.M && gn + 8 <= p.N) ? static_cast<int64_t>(gm) * p.N + gn : 0;
-        rres[i] = *reinterpret_cast<const uint4*>(p.residual + idx);
+        rres[i] = *reinterpret_cast<const uint4*>(residual + idx);
       }
     }
   }
@@ -568,7 +730,7 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
     if (gm >= p.M || gn >= p.N) continue;
     const uint16_t* t = T + row * TS + cc * 8;
     // destination of column gn (split: the output whose column range holds it)
-    uint16_t* o = p.out0;
+    uint16_t* o = out0;
     int32_t col = gn, ld = p.N, lim = p.N;  // lim: end of the destination's columns
     if constexpr (EPI == kI4Split) {
       if (gn < p.c1) {
@@ -603,73 +765,90 @@ __global__ __launch_bounds__((Shape<WF, NWN>::kThreads), NWN == 2 ? 2 : 1) void 
       // per element: the N edge, a chunk that straddles split outputs, unaligned rows
       for (int e = 0; e < 8 && gn + e < p.N; ++e) {
         int32_t ge = gn + e;
-        uint16_t* de = p.out0 + static_cast<int64_t>(gm) * p.N + ge;
+        uint16_t* de = out0 + static_cast<int64_t>(gm) * p.N + ge;
         if constexpr (EPI == kI4Split) {
-          if (ge < p.c1) de = p.out0 + static_cast<int64_t>(gm) * p.c1 + ge;
+          if (ge < p.c1) de = out0 + static_cast<int64_t>(gm) * p.c1 + ge;
           else if (ge < p.c2) de = p.out1 + static_cast<int64_t>(gm) * (p.c2 - p.c1) + (ge - p.c1);
           else de = p.out2 + static_cast<int64_t>(gm) * (p.N - p.c2) + (ge - p.c2);
         }
         uint16_t v = t[e];
         if constexpr (EPI == kI4Residual)
-          v = f32_to_bf16_bits(bf16_bits_to_f32(p.residual[static_cast<int64_t>(gm) * p.N + ge]) + bf16_bits_to_f32(v));
+          v = f32_to_bf16_bits(bf16_bits_to_f32(residual[static_cast<int64_t>(gm) * p.N + ge]) + bf16_bits_to_f32(v));
         *de = v;
       }
     }
   }
 }
 
-// Tiles of a launch with NWN waves along N.
-template <int EPI, int NWN>
+// Tiles of a launch.
+template <int WF, int EPI, int TILE>
 int64_t TilesOf(const I4Args& p) {
-  const int64_t tiles_m = CeilDiv(p.M, QBM);
-  constexpr int64_t BN = 64 * NWN;
-  return tiles_m * (EPI == kI4SiluMul ? p.ffn / (BN / 2) : CeilDiv(p.N, BN));
+  using S = Shape<WF, TILE>;
+  constexpr int64_t BN = S::kBN;
+  return CeilDiv(p.M, S::kBM) * (EPI == kI4SiluMul ? p.ffn / (BN / 2) : CeilDiv(p.N, BN));
 }
 
 constexpr int64_t kTicketRegion = 4096;               // bytes at the start of the workspace
 constexpr int64_t kMaxSplitTiles = kTicketRegion / 4;  // tiles of a launch that may split
 
-// Blocks of a shape that one CU holds at once, by LDS (160 KB per CU): two for the
-// 128-wide INT4 and INT8 tiles, one for the bf16 tile and for every 256-wide tile.
+// Blocks of a shape that one CU holds at once, by LDS (160 KB per CU): two for the 64-row
+// tiles and the 128 x 128 INT4 and INT8 ones, one for the others.
 constexpr int64_t kLdsPerCu = 160 * 1024;
-template <int WF, int NWN>
+template <int WF, int TILE>
 constexpr int BlocksPerCu() {
-  return kLdsPerCu / Shape<WF, NWN>::kLds > 1 ? static_cast<int>(kLdsPerCu / Shape<WF, NWN>::kLds) : 1;
+  return kLdsPerCu / Shape<WF, TILE>::kLds > 1 ? static_cast<int>(kLdsPerCu / Shape<WF, TILE>::kLds) : 1;
 }
 
-// Split-K count: the largest power of two <= 4 that keeps every split at >= 8 groups
-// and the launch within one round of resident blocks (bpc per CU).  Measured on the
-// 8B 512-row shapes with the 16-byte partial stores: q|k|v 2 splits (INT4 71 -> 58 us,
-// INT8 103 -> 64 us; bf16, one block per CU, unsplit), o 4 (INT4 44 -> 39 us, INT8
-// 60 -> 43 us; bf16 2), down 4 (bf16 2: 116 -> 109 us), gate/up unsplit (448 tiles
-// already fill the CUs; 2 splits 206 -> 232 us).
-int SplitsFor(int64_t tiles, int64_t groups, int64_t cus, int bpc) {
+// Split-K count: the largest power of two up to `most` that keeps every split at >= 8
+// groups (12 beyond 4 splits) and the launch within one round of resident blocks (bpc per
+// CU).  512 rows of the 8B o projection, INT4: 47 us unsplit by estimate, 36 us with 4
+// splits; 64 rows of its down projection: 24 us with 8 splits of 64 x 64 tiles, 54 us with
+// 4 of 128 x 128.
+int SplitsFor(int64_t tiles, int64_t groups, int64_t cus, int bpc, int most) {
   if (tiles > kMaxSplitTiles) return 1;
   int s = 1;
-  while (s < 4 && tiles * s * 2 <= bpc * cus && groups / (s * 2) >= 8) s *= 2;
+  while (s < most && tiles * s * 2 <= bpc * cus && groups / (s * 2) >= (s < 4 ? 8 : 12)) s *= 2;
   return s;
 }
+
+// 8 splits only for the small tiles (k of 12288 and more), 2 for the bf16 128 x 256 tile
+// (its 4-split launches are within 3% of two splits of 128 x 128 and take twice the
+// workspace).
+template <int WF, int TILE>
+constexpr int MaxSplits() {
+  return TILE == kT64 || TILE == kT64W ? 8 : TILE == kT256 && WF == AM_WF_BF16 ? 2 : 4;
+}
+constexpr int32_t kFewRows = 256;
 
 // Workspace layout: a fixed ticket region (one u32 per tile of a splitting launch),
 // then the partials.  The region's size does not depend on the launch's shape, so
 // launches of different shapes can share one workspace: no launch's partials land on
 // another launch's tickets.
 int64_t TicketBytes(int64_t) { return kTicketRegion; }
-template <int NWN>
+template <int WF, int TILE>
 int64_t PartialBytes(int64_t tiles, int splits) {
-  return splits > 1 ? tiles * splits * (2 * NWN) * (16 * 64 * 16) : 0;
+  using S = Shape<WF, TILE>;
+  return splits > 1 ? tiles * splits * S::kWaves * S::kPartWave * 4 : 0;
 }
 
-template <int WF, int EPI, int NWN>
+// Splits a launch of this tile runs with the given workspace.
+template <int WF, int EPI, int TILE>
+int SplitsOf(const I4Args& p, const void* ws, int64_t ws_bytes) {
+  if (ws == nullptr) return 1;
+  const int64_t tiles = TilesOf<WF, EPI, TILE>(p);
+  const int s = SplitsFor(tiles, p.K / p.group, DeviceCUs(), BlocksPerCu<WF, TILE>(), MaxSplits<WF, TILE>());
+  return s > 1 && TicketBytes(tiles) + PartialBytes<WF, TILE>(tiles, s) > ws_bytes ? 1 : s;
+}
+
+template <int WF, int EPI, int TILE>
 am_status_code LaunchMfma(I4Args p, void* ws, int64_t ws_bytes, hipStream_t s) {
-  using S = Shape<WF, NWN>;
+  using S = Shape<WF, TILE>;
   static const bool lds_ok =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mfma_kernel<WF, EPI, NWN>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mfma_kernel<WF, EPI, TILE>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds) == hipSuccess;
   if (!lds_ok) return SetLastError(AM_STATUS_INTERNAL, "gemm_i4: could not set the dynamic LDS size");
-  const int64_t tiles = TilesOf<EPI, NWN>(p);
-  int splits = ws != nullptr ? SplitsFor(tiles, p.K / p.group, DeviceCUs(), BlocksPerCu<WF, NWN>()) : 1;
-  if (splits > 1 && TicketBytes(tiles) + PartialBytes<NWN>(tiles, splits) > ws_bytes) splits = 1;
+  const int64_t tiles = TilesOf<WF, EPI, TILE>(p);
+  const int splits = SplitsOf<WF, EPI, TILE>(p, ws, ws_bytes);
   p.splits = splits;
   if (splits > 1) {
     p.tickets = static_cast<unsigned*>(ws);
@@ -679,23 +858,55 @@ am_status_code LaunchMfma(I4Args p, void* ws, int64_t ws_bytes, hipStream_t s) {
   static const char* const names[] = {"store", "residual", "split", "silu_mul", "qkv_rope_kv"};
   const char* fmt = WF == AM_WF_INT4 ? "i4" : WF == AM_WF_INT8 ? "i8" : "bf16";
   RecordLaunch(blocks, S::kThreads, S::kLds, "gemm_%s<%s,bn=%d,splits=%d>", fmt, names[EPI], S::kBN, splits);
-  hipLaunchKernelGGL((gemm_mfma_kernel<WF, EPI, NWN>), dim3(static_cast<unsigned>(blocks)), dim3(S::kThreads), S::kLds,
+  hipLaunchKernelGGL((gemm_mfma_kernel<WF, EPI, TILE>), dim3(static_cast<unsigned>(blocks)), dim3(S::kThreads), S::kLds,
                      s, p);
   AM_RETURN_IF_LAUNCH_FAILED("gemm_i4");
   return AM_STATUS_OK;
 }
 
-// Tile width per shape: the 256-wide tile when it still gives every CU a block.
-template <int EPI>
-bool WideI4(const I4Args& p) {
-  const int64_t tiles_m = CeilDiv(p.M, QBM);
-  const int64_t cols = EPI == kI4SiluMul ? 2 * static_cast<int64_t>(p.ffn) : p.N;
-  return (EPI != kI4SiluMul || p.ffn % 128 == 0) && tiles_m * CeilDiv(cols, 256) >= DeviceCUs();
+// ---- choice of the tile ----
+// Estimated time of a launch in us.  Compute: rounds of resident blocks, each a split's k
+// steps at the measured time of a 64-value step with the CU full (2048 x 28672 x 4096, the
+// 64 x 64 tile 2048 x 4096 x 4096, divided by rounds and steps); a last round that leaves
+// one block to a CU that holds two runs its steps in 0.62 of that.  Weights: read at about
+// 5 TB/s.  Split merge: every partial is stored at about 5 TB/s in all, and a tile's last
+// block reads all of them back at what one CU reads (75 GB/s).  On the 8B shapes from 20
+// to 2048 rows the estimates fall within a tenth to a fifth of the measured times and
+// order the tiles as measured, up to ties (512 rows, q|k|v INT4: 128 x 128 46 us, 128 x
+// 256 45 us, 256 x 256 55 us; estimated 48, 48, 63).
+//                                128x128 128x256 64x64  64x128 256x256
+constexpr float kStepUs[3][5] = {{1.20f, 1.13f, 0.46f, 0.73f, 2.05f},   // INT4, by Tile
+                                 {1.08f, 1.03f, 0.45f, 0.69f, 1.82f},   // INT8
+                                 {0.65f, 1.01f, 0.38f, 0.71f, 1.68f}};  // bf16
+template <int WF, int EPI, int TILE>
+float EstimateUs(const I4Args& p, const void* ws, int64_t ws_bytes) {
+  using S = Shape<WF, TILE>;
+  if (p.group % S::BK != 0) return 1e30f;
+  if (EPI == kI4SiluMul && p.ffn % (S::kBN / 2) != 0) return 1e30f;
+  constexpr float step = kStepUs[WF == AM_WF_INT4 ? 0 : WF == AM_WF_INT8 ? 1 : 2][TILE];
+  const int64_t cus = DeviceCUs(), bpc = BlocksPerCu<WF, TILE>(), tiles = TilesOf<WF, EPI, TILE>(p);
+  const int splits = SplitsOf<WF, EPI, TILE>(p, ws, ws_bytes);
+  const int64_t blocks = tiles * splits, slots = cus * bpc, rest = blocks % slots;
+  const float rounds = static_cast<float>(blocks / slots) + (rest == 0 ? 0.0f : rest <= cus && bpc > 1 ? 0.62f : 1.0f);
+  constexpr float tile = S::kBM * S::kBN * 4;
+  const float merge = splits > 1 ? 2.0f + static_cast<float>(splits + 1) * tile / 75e3f + static_cast<float>(blocks) * tile / 5e6f : 0.0f;
+  const float weights = static_cast<float>(p.N) * (p.K / QBK) * WRow<WF>::kBytes / 5e6f;
+  return std::max(rounds * static_cast<float>(p.K / QBK) / splits * step, weights) + merge;
 }
 
+// The tile with the smallest estimate.  The 64-row tiles take part up to 256 rows (above,
+// they read each weight more often than a launch of wider tiles of the same estimate).
 template <int WF, int EPI>
 am_status_code LaunchWF(const I4Args& p, void* ws, int64_t ws_bytes, hipStream_t s) {
-  return WideI4<EPI>(p) ? LaunchMfma<WF, EPI, 4>(p, ws, ws_bytes, s) : LaunchMfma<WF, EPI, 2>(p, ws, ws_bytes, s);
+  constexpr int kFew = EPI == kI4SiluMul ? kT64W : kT64;
+  const float few = p.M <= kFewRows ? EstimateUs<WF, EPI, kFew>(p, ws, ws_bytes) : 1e30f;
+  const float t128 = EstimateUs<WF, EPI, kT128>(p, ws, ws_bytes), t256 = EstimateUs<WF, EPI, kT256>(p, ws, ws_bytes),
+              big = EstimateUs<WF, EPI, kT256x256>(p, ws, ws_bytes);
+  const float best = std::min(std::min(few, t128), std::min(t256, big));
+  if (best == few) return LaunchMfma<WF, EPI, kFew>(p, ws, ws_bytes, s);
+  if (best == t256) return LaunchMfma<WF, EPI, kT256>(p, ws, ws_bytes, s);
+  if (best == big) return LaunchMfma<WF, EPI, kT256x256>(p, ws, ws_bytes, s);
+  return LaunchMfma<WF, EPI, kT128>(p, ws, ws_bytes, s);
 }
 
 // The weight format picks the kernel (p.group: the INT4 group, 128 otherwise).
@@ -741,15 +952,24 @@ int64_t GemmI4WorkspaceBytes(int64_t m, int64_t n, int64_t k, int64_t group) {
   if (m <= 0 || n <= 0 || k <= 0 || group <= 0 || k % group != 0) return 0;
   const int64_t cus = DeviceCUs();
   int64_t best = 0;
-  for (int nwn : {2, 4}) {
-    const int64_t tiles = CeilDiv(m, QBM) * CeilDiv(n, 64 * nwn);
-    const int bpc = nwn == 2 ? std::max({BlocksPerCu<AM_WF_INT4, 2>(), BlocksPerCu<AM_WF_INT8, 2>(),
-                                         BlocksPerCu<AM_WF_BF16, 2>()})
-                             : std::max({BlocksPerCu<AM_WF_INT4, 4>(), BlocksPerCu<AM_WF_INT8, 4>(),
-                                         BlocksPerCu<AM_WF_BF16, 4>()});
-    const int sp = SplitsFor(tiles, k / group, cus, bpc);
-    if (sp > 1)
-      best = std::max(best, TicketBytes(tiles) + (nwn == 2 ? PartialBytes<2>(tiles, sp) : PartialBytes<4>(tiles, sp)));
+  auto shape = [&](auto tile, auto fmt) {
+    constexpr int T = decltype(tile)::value, WF = decltype(fmt)::value;
+    using S = Shape<WF, T>;
+    const int64_t tiles = CeilDiv(m, S::kBM) * CeilDiv(n, S::kBN);
+    const int sp = SplitsFor(tiles, k / group, cus, BlocksPerCu<WF, T>(), MaxSplits<WF, T>());
+    if (sp > 1) best = std::max(best, TicketBytes(tiles) + PartialBytes<WF, T>(tiles, sp));
+  };
+  auto tile = [&](auto t) {
+    shape(t, std::integral_constant<int, AM_WF_INT4>{});
+    shape(t, std::integral_constant<int, AM_WF_INT8>{});
+    shape(t, std::integral_constant<int, AM_WF_BF16>{});
+  };
+  tile(std::integral_constant<int, kT128>{});
+  tile(std::integral_constant<int, kT256>{});
+  tile(std::integral_constant<int, kT256x256>{});
+  if (m <= kFewRows) {
+    tile(std::integral_constant<int, kT64>{});
+    tile(std::integral_constant<int, kT64W>{});
   }
   return best;
 }

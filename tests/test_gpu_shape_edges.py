@@ -13,8 +13,8 @@ if not torch.cuda.is_available():  # pragma: no cover
 
 import aethermind_amd.native as N  # noqa: E402
 import oracle_lib as O  # noqa: E402
-from gpu_util import bf16_dev, bits_host, dev, empty, host, p, pack_weight, stream  # noqa: E402
-from test_gpu_decode_shapes import act_rows, bf16_rne_bits, close, launched, rbf  # noqa: E402
+from gpu_util import bf16_dev, dev, empty, host, p, pack_weight, stream  # noqa: E402
+from test_gpu_decode_shapes import act_rows, bf16_rne_bits, launched, rbf  # noqa: E402
 
 L = N.lib()
 
@@ -64,3 +64,71 @@ def test_linear_f32_rows(m, n, k):
     L.call("am_gfx950_linear", N.LinearArgs(p(xd), 0, m, dw, p(rd), 0, p(rd), 0), stream())
     assert (np.abs(host(rd) - (ref + res)) <= bar + 2.0 ** -23 * np.abs(ref + res)).all()
     del keep
+
+
+# (m, n, k, group): rows and columns on both sides of the 64-, 128- and 256-row tiles of
+# every weight format, one k step, an odd number of groups, groups of one, two and four
+# 64-value steps
+TILE_SHAPES = [(1, 64, 128, 128), (65, 72, 384, 128), (256, 4104, 640, 128), (257, 16392, 384, 128),
+               (513, 28680, 512, 256), (300, 8200, 1024, 64), (1030, 6152, 2048, 128)]
+
+
+@pytest.mark.parametrize("shape", TILE_SHAPES)
+@pytest.mark.parametrize("fmt", [N.AM_WF_INT4, N.AM_WF_INT8, N.AM_WF_BF16])
+def test_prefill_gemm_tiles(shape, fmt):
+    """Every element against the fp64 product of the dequantized weights.  Bar: half a
+    bf16 ulp of the result (2^-8 relative, generously) and k * 2^-24 of the summed
+    magnitudes for the fp32 sums."""
+    m, n, k, group = shape
+    rng = np.random.default_rng(m + n)
+    w = rbf(rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02))
+    if group <= k // 2:
+        w[::7, :group] = 0.0  # whole groups of zero scale
+        w[3::7, group:2 * group] *= 1e-3  # neighbouring groups of very different scales
+    dw, keep = pack_weight(w, fmt, group)
+    if fmt == N.AM_WF_INT4:
+        pk, sc = O.quant_int4(w, group)
+        w = O.dequant_int4(pk, sc, k, group)
+    elif fmt == N.AM_WF_INT8:
+        w = O.dequant_int8(*O.quant_int8(w))
+    x = act_rows(7, m, k)
+    xd, wd = bf16_dev(bf16_rne_bits(x)), dev(w)
+    xt = dev(x).double()
+    ref, mag = xt @ wd.double().T, xt.abs() @ wd.double().abs().T
+    nbytes = L.am_gfx950_gemm_workspace_bytes(m, n, k, group if fmt == N.AM_WF_INT4 else 128)
+    ws = torch.zeros(max(nbytes, 16), dtype=torch.uint8, device="cuda")
+    for use_ws in (False, True):
+        out = empty((m, n), torch.bfloat16)
+        args = N.LinearArgs(p(xd), N.AM_DT_BF16, m, dw, p(out), N.AM_DT_BF16, None, 2)
+        if use_ws and nbytes:
+            args.workspace, args.workspace_bytes = p(ws), nbytes
+        L.call("am_gfx950_linear", args, stream())
+        err = (out.double() - ref).abs()
+        bar = ref.abs() * 2.0 ** -8 + mag * (k * 2.0 ** -24) + 1e-30
+        assert bool((err <= bar).all()), (launched(), float((err - bar).max()))
+    del keep
+
+
+def test_prefill_gemm_zero_scale_groups():
+    """INT4 groups whose scale is zero but whose codes are not add nothing."""
+    m, n, k, group = 70, 256, 512, 128
+    rng = np.random.default_rng(5)
+    codes = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    sc = (rng.random((n, k // group), dtype=np.float32) * 0.1).astype(np.float16)
+    sc[::2, 0] = 0
+    sc[::3, 2] = 0
+    sc[5, :] = 0
+    logical, scales = dev(codes), dev(sc.view(np.int16))
+    data = torch.zeros(n * k // 2, dtype=torch.uint8, device="cuda")
+    dsc = torch.zeros(n * (k // group), dtype=torch.int16, device="cuda")
+    dw = N.Weight(p(data), p(dsc), n, k, N.AM_WF_INT4, group)
+    L.call("am_gfx950_pack_int4", N.PackInt4Args(p(logical), p(scales), dw), stream())
+    q = np.stack([codes & 15, codes >> 4], -1).reshape(n, k).astype(np.int32)
+    w = np.where(q > 7, q - 16, q) * np.repeat(sc.astype(np.float64), group, 1)
+    x = act_rows(8, m, k)
+    xd = bf16_dev(bf16_rne_bits(x))
+    out = empty((m, n), torch.bfloat16)
+    L.call("am_gfx950_linear", N.LinearArgs(p(xd), N.AM_DT_BF16, m, dw, p(out), N.AM_DT_BF16, None, 2), stream())
+    ref = x.astype(np.float64) @ w.T
+    bar = np.abs(ref) * 2.0 ** -8 + k * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + 1e-12
+    assert (np.abs(out.double().cpu().numpy() - ref) <= bar).all()
