@@ -27,6 +27,7 @@
 
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <mutex>
@@ -47,6 +48,7 @@ struct AttnArgs {
   int64_t cbs;  // cache batch stride (elements)
   int32_t splits;
   int32_t min_per_split;  // fewest positions one split block handles
+  int32_t short_splits;   // decode kernel: most splits of a context below kDecLong
   float scale;  // log2(e) / sqrt(d)
   float* part;
   unsigned* tickets;  // [rows][hkv], zero between calls
@@ -511,6 +513,7 @@ __global__ __launch_bounds__(kWaves * 64) void attention_kernel(AttnArgs p) {
 //   * The per-wave states are merged in LDS, and split blocks merge through the same
 //     records and ticket as the general kernel.
 constexpr int kDecWaves = 4;
+constexpr int64_t kDecLong = 4096;
 // Split policy of the decode kernel, measured on MI355X with a cold cache (the layer's
 // K/V evicted by the weight stream, as in decode) and in the replayed decode graph: at
 // least 64 positions per split block and at most 8 split blocks per (row, kv head)
@@ -536,15 +539,20 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(AttnArgs p) {
   const int j = lane & 15, h = lane >> 4;
   typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
   typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-  const int64_t qr = blockIdx.z;
+  // Grid (splits, kv heads, rows), or (kv heads, rows, splits) where a context may use
+  // fewer splits than the grid has: the live blocks then come first and spread over the
+  // XCDs (block i runs on XCD i mod 8; 16 rows at contexts 400-777, 2 of 4 splits live: 18.4
+  // us with the splits first, 12.6 us).
+  const bool live_first = p.short_splits < p.splits;
+  const int64_t qr = live_first ? blockIdx.y : blockIdx.z;
   const int64_t b = qr / p.seq, s = qr % p.seq;
-  const int64_t g = blockIdx.y;
-  const int split = blockIdx.x;
+  const int64_t g = live_first ? blockIdx.x : blockIdx.y;
+  const int split = live_first ? blockIdx.z : blockIdx.x;
   const int64_t n_keys = row_keys(p, b, s);
   // Slices are whole 32-position steps (a step then never straddles two cache blocks):
   // the slice length is rounded up to 32 and the live split count follows from it,
   // the same in every block of the (row, kv head).
-  const int64_t ns0 = live_splits(n_keys, p.splits, p.min_per_split);
+  const int64_t ns0 = live_splits(n_keys, n_keys < kDecLong ? p.short_splits : p.splits, p.min_per_split);
   const int64_t per = (((n_keys + ns0 - 1) / ns0) + 31) & ~int64_t{31};
   const int64_t nsplit = (n_keys + per - 1) / per;
   if (split >= nsplit) return;  // surplus block for this context
@@ -1140,10 +1148,10 @@ template <int D, int NW>
 am_status_code LaunchDecode(int64_t G, dim3 grid, const AttnArgs& a, hipStream_t s) {
   if constexpr (NW == kDecWaves)
     RecordLaunch(GridBlocks(grid), NW * 64, 0, "attention_decode<d=%d,g=%d,splits=%u>", D, static_cast<int>(G),
-                 grid.x);
+                 static_cast<unsigned>(a.splits));
   else
     RecordLaunch(GridBlocks(grid), NW * 64, 0, "attention_decode<d=%d,g=%d,splits=%u,waves=%d>", D,
-                 static_cast<int>(G), grid.x, NW);
+                 static_cast<int>(G), static_cast<unsigned>(a.splits), NW);
   const dim3 block(NW * 64);
   switch (G) {
     case 1: LaunchTimed(attention_decode_kernel<D, 1, NW>, grid, block, s, a); break;
@@ -1303,10 +1311,25 @@ extern "C" am_status_code am_gfx950_attention(const am_gfx950_attention_args* a,
     // decode: MFMA kernel; an explicit split request is honoured down to 32 positions
     p.min_per_split = a->num_splits > 0 ? 32 : kDecMinPerSplit;
     if (a->num_splits <= 0 && p.splits > kDecMaxSplits) p.splits = kDecMaxSplits;
-    const dim3 grid(static_cast<unsigned>(p.splits), static_cast<unsigned>(a->hkv), static_cast<unsigned>(batch));
-    // Grids that give every CU a block (batched long contexts) run 8-wave blocks, two
-    // waves per SIMD: twice the K/V loads in flight per CU, merged in LDS.
-    if (a->num_splits <= 0 && GridBlocks(grid) >= DeviceCUs())
+    // Grids that give every CU a block run 8-wave blocks, two waves per SIMD: twice the
+    // K/V loads in flight per CU, merged in LDS.  One such block fits a CU and more run in
+    // rounds, so the splits are cut to one round of blocks: 16 rows at contexts 400-777
+    // 24.0 -> 12.0 us, 1000-2000 32.4 -> 23.3, 4000-8000 84.0 -> 81.6; 5 rows at 4000-8000
+    // 35.5 -> 30.6.  Where one round leaves more than an eighth of the CUs idle and two
+    // rounds do not, contexts of kDecLong positions take two (12 rows at 4000-8000: 65.1
+    // us with 8 splits, 67.0 in one round, 64.3 in two).
+    const int64_t pairs = a->hkv * batch, cus = DeviceCUs();
+    const bool wide = a->num_splits <= 0 && pairs * p.splits >= cus;
+    p.short_splits = p.splits;
+    if (wide) {
+      const int64_t one = std::max<int64_t>(1, std::min<int64_t>(p.splits, cus / pairs));
+      const int64_t two = std::max<int64_t>(1, std::min<int64_t>(p.splits, 2 * cus / pairs));
+      p.short_splits = static_cast<int32_t>(one);
+      p.splits = static_cast<int32_t>(8 * one * pairs < 7 * cus && 8 * two * pairs >= 14 * cus ? two : one);
+    }
+    const unsigned ns = static_cast<unsigned>(p.splits), nh = static_cast<unsigned>(a->hkv), nb = static_cast<unsigned>(batch);
+    const dim3 grid = p.short_splits < p.splits ? dim3(nh, nb, ns) : dim3(ns, nh, nb);
+    if (wide)
       return a->head_dim == 128 ? LaunchDecode<128, 8>(G, grid, p, s) : LaunchDecode<64, 8>(G, grid, p, s);
     return a->head_dim == 128 ? LaunchDecode<128, kDecWaves>(G, grid, p, s)
                               : LaunchDecode<64, kDecWaves>(G, grid, p, s);

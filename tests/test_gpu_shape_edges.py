@@ -2,6 +2,8 @@
 next to an edge of the variant it reaches, against the CPU oracle (or numpy for exact
 results)."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -132,3 +134,42 @@ def test_prefill_gemm_zero_scale_groups():
     ref = x.astype(np.float64) @ w.T
     bar = np.abs(ref) * 2.0 ** -8 + k * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + 1e-12
     assert (np.abs(out.double().cpu().numpy() - ref) <= bar).all()
+
+
+@pytest.mark.parametrize("B,hkv", [(16, 8), (12, 8), (9, 8), (5, 8), (64, 8), (24, 2)])
+@pytest.mark.parametrize("paged", [False, True])
+def test_attention_decode_split_rounds(B, hkv, paged):
+    """Batched decode grids whose splits are cut to one or two rounds of blocks (and more
+    (row, head) pairs than CUs): contexts from one position to past the long-context
+    threshold side by side, against fp64 attention.  Twice on one workspace."""
+    g, d, cap = 4, 128, 4608
+    hq = g * hkv
+    rng = np.random.default_rng(B)
+    lens = [1, 31, 64, 65, 777, 4095, 4096, 4097, 4608]
+    pos = np.array([lens[i % len(lens)] - 1 for i in range(B)], np.int64)
+    k, v = (torch.randn((B, hkv, cap, d), device="cuda", generator=torch.Generator("cuda").manual_seed(s)).to(torch.bfloat16)
+            for s in (B, B + 1))
+    q = torch.randn((B, hq * d), device="cuda", generator=torch.Generator("cuda").manual_seed(3)).to(torch.bfloat16)
+    kd, vd, pages = k, v, None
+    if paged:
+        per = cap // 64
+        table = torch.from_numpy(rng.permutation(B * per).astype(np.int32)).cuda().view(B, per)
+        kd, vd = (torch.empty((B * per, hkv, 64, d), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        for src, dst in ((k, kd), (v, vd)):
+            dst[table.long().view(-1)] = src.view(B, hkv, per, 64, d).transpose(1, 2).reshape(B * per, hkv, 64, d)
+        pages = C.pointer(N.KvPages(p(table), 64, per, B * per, None))
+    posd = dev(pos)
+    wsb = L.am_gfx950_attention_workspace_bytes(B, 1, hq, hkv, d, cap, 0)
+    ws = torch.zeros(wsb, dtype=torch.uint8, device="cuda")
+    for _ in range(2):
+        out = empty((B, hq * d), torch.bfloat16)
+        L.call("am_gfx950_attention", N.AttentionArgs(p(q), p(kd), p(vd), p(out), 1, hq, hkv, d, cap, 0, p(posd), B,
+                                                      hkv * cap * d, 1, 0, p(ws), wsb, pages), stream())
+        for r in range(B):
+            n = int(pos[r]) + 1
+            kr, vr = (t[r, :, :n].double().repeat_interleave(g, 0) for t in (k, v))
+            sc = (kr * q[r].double().view(hq, 1, d)).sum(-1) / d ** 0.5
+            ref = (torch.softmax(sc, -1).unsqueeze(-1) * vr).sum(1).view(-1)
+            err = (out[r].double() - ref).abs()
+            # a bf16 rounding of the output and P in bf16 hi + lo (2^-16 of the row's largest value)
+            assert bool((err <= ref.abs() * 2.0 ** -8 + 2.0 ** -15 * vr.abs().max()).all()), (r, n)
