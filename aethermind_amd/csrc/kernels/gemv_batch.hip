@@ -76,11 +76,6 @@ template <> struct BFmt<AM_WF_BF16> { static constexpr int ks = 32, mi = 1; };
 template <> struct BFmt<AM_WF_INT8> { static constexpr int ks = 64, mi = 2; };
 template <> struct BFmt<AM_WF_INT4> { static constexpr int ks = 128, mi = 4; };
 
-__device__ __forceinline__ uint32_t pack_small_ints(float lo, float hi) {
-  // small integers: the bf16 encoding is the top half of the fp32 bits
-  return (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
-}
-
 // B operand of MFMA i from the lane's 16-byte weight slice (k values 8i..8i+7 of it)
 template <int WF>
 __device__ __forceinline__ bf16x8_t w_operand(const u32x4_t& v, int i, uint32_t mask, uint32_t magic) {
@@ -90,13 +85,13 @@ __device__ __forceinline__ bf16x8_t w_operand(const u32x4_t& v, int i, uint32_t 
   } else if constexpr (WF == AM_WF_INT8) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const uint32_t wd = v[2 * i + h];
-      const float q0 = static_cast<float>(wd & 0xFFu) - 128.0f;
-      const float q1 = static_cast<float>((wd >> 8) & 0xFFu) - 128.0f;
-      const float q2 = static_cast<float>((wd >> 16) & 0xFFu) - 128.0f;
-      const float q3 = static_cast<float>(wd >> 24) - 128.0f;
-      o[2 * h] = pack_small_ints(q0, q1);
-      o[2 * h + 1] = pack_small_ints(q2, q3);
+      // q + 128 with the top bit flipped is q in two's complement: signed byte
+      // conversions, whose fp32 top halves are the bf16 encodings of small integers
+      const uint32_t wd = v[2 * i + h] ^ 0x80808080u;
+      const float q0 = static_cast<float>(static_cast<int8_t>(wd)), q1 = static_cast<float>(static_cast<int8_t>(wd >> 8));
+      const float q2 = static_cast<float>(static_cast<int8_t>(wd >> 16)), q3 = static_cast<float>(static_cast<int8_t>(wd >> 24));
+      o[2 * h] = __builtin_amdgcn_perm(__float_as_uint(q1), __float_as_uint(q0), 0x07060302u);
+      o[2 * h + 1] = __builtin_amdgcn_perm(__float_as_uint(q3), __float_as_uint(q2), 0x07060302u);
     }
   } else {
     const uint32_t wd = v[i];
@@ -138,9 +133,11 @@ __device__ __forceinline__ int tile_row(const BatchArgs& p, int u, int tt) {
   }
 }
 
-// R: k steps of loads in flight per wave (per tile)
-template <int WF, int EPI, bool NORM, int TPB, int R>
+// R: k steps of loads in flight per wave (per tile).  XG: the token rows are not staged
+// in LDS; each wave loads the A operands of its own steps beside the weights.
+template <int WF, int EPI, bool NORM, int TPB, int R, bool XG>
 __global__ __launch_bounds__(kBWaves * 64) void gemv_batch_kernel(BatchArgs p) {
+  static_assert(!(XG && NORM), "normalised rows are staged");
   constexpr int NW = kBWaves, NT = NW * 64;
   constexpr int KS = BFmt<WF>::ks, MI = BFmt<WF>::mi;
   extern __shared__ __align__(16) uint8_t bsm[];
@@ -151,7 +148,7 @@ __global__ __launch_bounds__(kBWaves * 64) void gemv_batch_kernel(BatchArgs p) {
   const int XR = K + 8;                        // LDS row stride (elements)
   const int cnt = ((S + NW - 1) / NW + R - 1) / R * R;  // steps per wave and unit (padded)
   uint16_t* xs = reinterpret_cast<uint16_t*>(bsm);
-  float* red = reinterpret_cast<float*>(bsm + ((static_cast<size_t>(rows) * XR * 2 + 15) & ~size_t{15}));
+  float* red = reinterpret_cast<float*>(bsm + (XG ? 0 : ((static_cast<size_t>(rows) * XR * 2 + 15) & ~size_t{15})));
   // [NW][TPB][64][4]
   float* nred = red + NW * TPB * 256;                   // [NW][16]
   // INT4 group scales of a unit as fp32, double-buffered: [2][TPB][16 rows][S + 1]
@@ -183,8 +180,10 @@ __global__ __launch_bounds__(kBWaves * 64) void gemv_batch_kernel(BatchArgs p) {
     return reinterpret_cast<u32x4_t*>(xs + b * XR + 8 * (e - b * pieces));
   };
   u32x4_t xv[XB];
+  if constexpr (!XG) {
 #pragma unroll
-  for (int j = 0; j < XB; ++j) xv[j] = *xsrc(tid + NT * j);
+    for (int j = 0; j < XB; ++j) xv[j] = *xsrc(tid + NT * j);
+  }
   const uint4* nw = reinterpret_cast<const uint4*>(p.norm_w);
   uint4 nw0 = make_uint4(0u, 0u, 0u, 0u);
   if constexpr (NORM) nw0 = nw[min(tid, pieces - 1)];
@@ -225,6 +224,8 @@ __global__ __launch_bounds__(kBWaves * 64) void gemv_batch_kernel(BatchArgs p) {
   // unconditional: a conditional refill makes the compiler's memory-counter waits
   // conservative at the loop head.
   u32x4_t wv[R][TPB];
+  u32x4_t xg[R][XG ? MI : 1];  // XG: the A operands of the slot's step (lanes past the batch read row 0)
+  const uint16_t* xg_src = p.x + (fl < rows ? fl : 0) * p.x_stride + g * (KS / 4);
   const uint8_t* tail_src = reinterpret_cast<const uint8_t*>(p.x) + (lane * 16) % (rows * K * 2);
   // lane's row pointers of the tiles of a unit (computed once per unit)
   auto row_ptrs = [&](const int (&rb)[TPB], bool tail, const uint8_t* (&wp)[TPB]) {
@@ -237,6 +238,11 @@ __global__ __launch_bounds__(kBWaves * 64) void gemv_batch_kernel(BatchArgs p) {
 #pragma unroll
     for (int tt = 0; tt < TPB; ++tt)
       wv[r][tt] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp[tt] + off));
+    if constexpr (XG) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+        xg[r][i] = *reinterpret_cast<const u32x4_t*>(xg_src + min(wave + NW * t, S - 1) * KS + 8 * i);
+    }
   };
   const int grid = gridDim.x;
   int u = blockIdx.x;
@@ -252,13 +258,15 @@ __global__ __launch_bounds__(kBWaves * 64) void gemv_batch_kernel(BatchArgs p) {
   // ---- prologue: token rows -> LDS (bf16), RMSNorm'd when NORM ----
   // stores are unconditional (clamped): a store under a branch would pull its load
   // into the branch, behind a wait for every weight load issued above
+  if constexpr (!XG) {
 #pragma unroll
-  for (int j = 0; j < XB; ++j) *xdst(tid + NT * j) = xv[j];
-  for (int e0 = XB * NT; e0 < tp; e0 += XB * NT) {  // more than XB pieces per thread
+    for (int j = 0; j < XB; ++j) *xdst(tid + NT * j) = xv[j];
+    for (int e0 = XB * NT; e0 < tp; e0 += XB * NT) {  // more than XB pieces per thread
 #pragma unroll
-    for (int j = 0; j < XB; ++j) xv[j] = *xsrc(e0 + tid + NT * j);
+      for (int j = 0; j < XB; ++j) xv[j] = *xsrc(e0 + tid + NT * j);
 #pragma unroll
-    for (int j = 0; j < XB; ++j) *xdst(e0 + tid + NT * j) = xv[j];
+      for (int j = 0; j < XB; ++j) *xdst(e0 + tid + NT * j) = xv[j];
+    }
   }
   store_scales(0);
   if constexpr (NORM) {
@@ -328,7 +336,9 @@ __global__ __launch_bounds__(kBWaves * 64) void gemv_batch_kernel(BatchArgs p) {
         bf16x8_t xa[MI];
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
-          const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(xrow + s * KS + 8 * i);
+          bf16x8_t v;
+          if constexpr (XG) v = __builtin_bit_cast(bf16x8_t, xg[r][i]);
+          else v = *reinterpret_cast<const bf16x8_t*>(xrow + s * KS + 8 * i);
           xa[i] = xrow_ok ? v : bf16x8_t{};
         }
         // INT4: the step's MFMA sums start at -136 * sum(x) of each token row, itself an
@@ -450,9 +460,12 @@ __global__ __launch_bounds__(kBWaves * 64) void gemv_batch_kernel(BatchArgs p) {
 }
 
 // ---- host ----
-template <int WF, int EPI, bool NORM, int TPB, int R>
+constexpr size_t kBatchLds = 160 * 1024;  // of one CU
+size_t BatchRowBytes(int64_t k, int64_t rows) { return (static_cast<size_t>(rows) * (k + 8) * 2 + 15) & ~size_t{15}; }
+
+template <int WF, int EPI, bool NORM, int TPB, int R, bool XG>
 am_status_code LaunchBatch(const BatchArgs& a, size_t lds, hipStream_t s) {
-  auto fn = gemv_batch_kernel<WF, EPI, NORM, TPB, R>;
+  auto fn = gemv_batch_kernel<WF, EPI, NORM, TPB, R, XG>;
   static thread_local size_t cached_lds = 0;
   static thread_local int cached_blocks = 0;
   if (cached_lds != lds) {
@@ -466,8 +479,8 @@ am_status_code LaunchBatch(const BatchArgs& a, size_t lds, hipStream_t s) {
     cached_lds = lds;
   }
   const int64_t blocks = std::min<int64_t>(a.units, static_cast<int64_t>(DeviceCUs()) * cached_blocks);
-  RecordLaunch(blocks, kBWaves * 64, static_cast<int32_t>(lds), "gemv_batch<wf=%d,epi=%d,norm=%d,tpb=%d,r=%d>", WF, EPI,
-               NORM ? 1 : 0, TPB, R);
+  RecordLaunch(blocks, kBWaves * 64, static_cast<int32_t>(lds), "gemv_batch<wf=%d,epi=%d,norm=%d,tpb=%d,r=%d%s>", WF, EPI,
+               NORM ? 1 : 0, TPB, R, XG ? ",xg" : "");
   LaunchTiming& lt = ThreadLaunchTiming();
   if (lt.start != nullptr) {
     hipExtLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks)), dim3(kBWaves * 64), lds, s, lt.start, lt.stop, 0,
@@ -484,11 +497,15 @@ am_status_code LaunchBatch(const BatchArgs& a, size_t lds, hipStream_t s) {
 // (long rows); paired units (two loads per step) and short rows keep 4.
 template <int WF, int EPI, bool NORM, int TPB>
 am_status_code LaunchBatchR(const BatchArgs& a, size_t lds, hipStream_t s) {
+  if constexpr (TPB == 1 && !NORM) {
+    // rows that do not fit LDS together: one launch that reads them beside the weights
+    if (lds > kBatchLds) return LaunchBatch<WF, EPI, NORM, TPB, WF == AM_WF_BF16 ? 8 : 4, true>(a, lds - BatchRowBytes(a.k, a.rows), s);
+  }
   if constexpr (TPB == 1) {
     const int S = a.k / BFmt<WF>::ks;
-    if ((S + kBWaves - 1) / kBWaves >= 8) return LaunchBatch<WF, EPI, NORM, TPB, 8>(a, lds, s);
+    if ((S + kBWaves - 1) / kBWaves >= 8) return LaunchBatch<WF, EPI, NORM, TPB, 8, false>(a, lds, s);
   }
-  return LaunchBatch<WF, EPI, NORM, TPB, 4>(a, lds, s);
+  return LaunchBatch<WF, EPI, NORM, TPB, 4, false>(a, lds, s);
 }
 
 template <int EPI, bool NORM, int TPB>
@@ -505,7 +522,7 @@ bool Aligned16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15u) ==
 // LDS of one block for `rows` token rows: the rows (bf16, padded by 16 bytes), the
 // per-wave partial tiles, 1/rms per row and, for INT4, the unit's group scales.
 size_t BatchLdsOf(const am_gfx950_weight& w, int64_t rows, int tpb) {
-  size_t b = (static_cast<size_t>(rows) * (w.k + 8) * 2 + 15) & ~size_t{15};
+  size_t b = BatchRowBytes(w.k, rows);
   b += static_cast<size_t>(kBWaves) * tpb * 256 * 4 + kBWaves * 16 * 4;
   if (w.format == AM_WF_INT4) b += static_cast<size_t>(2) * tpb * 16 * (w.k / 128 + 1) * 4;
   return b;
@@ -514,7 +531,7 @@ size_t BatchLdsOf(const am_gfx950_weight& w, int64_t rows, int tpb) {
 // Most token rows (up to 16) whose block fits the 160 KB of LDS (0: not even one).
 int64_t BatchRowsFit(const am_gfx950_weight& w, int tpb) {
   for (int64_t r = kBatchMaxRows; r >= 1; --r)
-    if (BatchLdsOf(w, r, tpb) <= 160 * 1024) return r;
+    if (BatchLdsOf(w, r, tpb) <= kBatchLds) return r;
   return 0;
 }
 
@@ -550,12 +567,16 @@ am_status_code PrepareBatch(const am_gfx950_weight& w, int64_t rows, const void*
 }
 
 // Runs launch(args, lds) over groups of token rows small enough for one block's LDS
-// (every group re-reads the weights): the k = 14336 down projection of the 8B shape
-// fits 5 rows of 14336 bf16 values; shorter rows fit all 16.  off(args, g0) moves the
-// group's row pointers (token rows, outputs, residuals, positions) to row g0.
+// (every group re-reads the weights; 16 rows of the 8B shapes' 4096 values fit).  off(args,
+// g0) moves the group's row pointers (outputs, positions) to row g0.  Rows that are only
+// multiplied (one tile per unit, no norm) run as one launch whatever their length: past
+// the LDS the kernel reads them from memory (XG).  The 8B down projection (k = 14336, 5
+// rows fit), INT4 / INT8 / bf16: 8 rows 28.3 / 35.7 / 62.2 -> 19.8 / 20.2 / 33.6 us, 16 rows
+// 56.3 / 70.1 / 122.7 -> 26.5 / 25.6 / 42 us.  Rows that fit stay in LDS (4 rows INT4
+// 14.4 us against 16.9).
 template <class Launch, class Offset>
 am_status_code ForRowGroups(const BatchArgs& a, const am_gfx950_weight& w, int tpb, Launch launch, Offset off) {
-  const int64_t per = std::min<int64_t>(a.rows, BatchRowsFit(w, tpb));
+  const int64_t per = tpb == 1 && a.norm_w == nullptr ? a.rows : std::min<int64_t>(a.rows, BatchRowsFit(w, tpb));
   for (int64_t g0 = 0; g0 < a.rows; g0 += per) {
     BatchArgs ga = a;
     ga.rows = static_cast<int32_t>(std::min<int64_t>(per, a.rows - g0));

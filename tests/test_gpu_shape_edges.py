@@ -173,3 +173,33 @@ def test_attention_decode_split_rounds(B, hkv, paged):
             err = (out[r].double() - ref).abs()
             # a bf16 rounding of the output and P in bf16 hi + lo (2^-16 of the row's largest value)
             assert bool((err <= ref.abs() * 2.0 ** -8 + 2.0 ** -15 * vr.abs().max()).all()), (r, n)
+
+
+@pytest.mark.parametrize("m,n,k", [(6, 4096, 14336), (16, 40, 14336), (9, 17, 16384), (16, 128, 5632)])
+@pytest.mark.parametrize("fmt", [N.AM_WF_INT4, N.AM_WF_INT8, N.AM_WF_BF16])
+def test_batched_rows_past_lds(m, n, k, fmt):
+    """Token rows that do not fit one block's LDS together run as one launch: Linear + Add
+    in place and the fp32 store, against the fp64 product of the dequantized weights."""
+    rng = np.random.default_rng(m + n)
+    w = rbf(rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02))
+    dw, keep = pack_weight(w, fmt)
+    if fmt == N.AM_WF_INT4:
+        pk, sc = O.quant_int4(w, 128)
+        w = O.dequant_int4(pk, sc, k, 128)
+    elif fmt == N.AM_WF_INT8:
+        w = O.dequant_int8(*O.quant_int8(w))
+    x, h = act_rows(9, m, k), act_rows(10, m, n)
+    xd, hd = bf16_dev(bf16_rne_bits(x)), bf16_dev(bf16_rne_bits(h))
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    sums = k * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T)
+    if fmt == N.AM_WF_INT4:
+        sums = sums * 20  # codes enter offset by 136: the partial sums reach 136 / 7 of the products'
+    L.call("am_gfx950_fused_linear_residual", N.FusedLinearResidualArgs(p(xd), dw, p(hd), N.AM_DT_BF16, m), stream())
+    assert launched().endswith(",xg>"), launched()
+    got = hd.view(torch.bfloat16).view(m, n).double().cpu().numpy()
+    bar = (np.abs(ref) + np.abs(ref + h)) * 2.0 ** -8 + sums
+    assert (np.abs(got - (ref + h)) <= bar).all()
+    out = empty((m, n), torch.float32)
+    L.call("am_gfx950_linear", N.LinearArgs(p(xd), N.AM_DT_BF16, m, dw, p(out), N.AM_DT_F32, None, 3), stream())
+    assert (np.abs(host(out) - ref) <= sums + 1e-30).all()
+    del keep
