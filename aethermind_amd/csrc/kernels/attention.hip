@@ -748,8 +748,8 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(AttnArgs p) {
 // with CG column groups of 16 MFMA columns (16/G positions x the G query heads of the
 // kv group), so a K/V load serves G heads and NW*CG*16/G positions.  The block walks
 // the key positions up to its last query's position in tiles of 32:
-//   * Tile t+2 is loaded into registers while tile t is computed and tile t+1 waits in
-//     LDS (two-deep prefetch; a tile is one cache block lookup, tiles start at
+//   * The next tile is loaded into registers while this one is computed, and stored into
+//     the other LDS buffer after it (a tile is one cache block lookup, tiles start at
 //     multiples of 32).  K is stored row-major and V transposed (V^T[d][key]); both are
 //     XOR-swizzled in 16-byte slots, so the operand reads below are conflict-free.
 //   * Scores S^T = K Q^T on v_mfma_f32_16x16x32_bf16 with the key rows of score tile tt
@@ -759,8 +759,8 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(AttnArgs p) {
 //     for output tile dt is V^T[16 dt + j][8h .. 8h+7], one 16-byte LDS read.  K and V
 //     operands are read once per wave and shared by the wave's column groups.
 //   * The causal mask is per column (key <= the column's position, key < the chunk
-//     end), the online softmax is base 2 per column (scores pre-scaled by
-//     log2(e)/sqrt(d)), P is split into bf16 hi + lo for the P V product.  Within a
+//     end), the online softmax is base 2 per column (the scale log2(e)/sqrt(d) is applied
+//     in the exponent's fma), P is split into bf16 hi + lo for the P V product.  Within a
 //     key group waves own distinct queries: each wave normalises its columns and
 //     writes them.
 // Blocks are numbered kv head fastest: block b runs on XCD b % 8, so with 8 kv heads
@@ -769,9 +769,17 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(AttnArgs p) {
 // first).
 // KS = 2 runs two groups of NW waves over the same queries: group k takes the key
 // tiles t with t % 2 == k through its own LDS buffers, and at the end the second
-// group's softmax states are merged into the first's through LDS.  A block then keeps
-// two waves per SIMD busy on half the tiles each, for launches that give a CU only one
-// 4-wave block.
+// group's softmax states are merged into the first's through LDS, one column group at a
+// time.  A block then keeps two waves per SIMD busy on half the tiles each: every shape
+// of 4 query waves runs so, and the shape of 8 has two waves per SIMD already.
+// What bounds it: the VALU operations of the softmax and the hi/lo split, which the MFMAs
+// of a SIMD's other wave hide only in part, and for short launches the chain of one tile.
+// Attention of 32 q / 8 kv heads, d = 128, one register set and a rolled tile loop, the
+// scale in the fma and two P values per conversion (before -> now, us): 300 positions
+// 13.4 -> 12.9; 512 18.4 -> 17.6; 1000 61.8 -> 41.3 and at 3000 keys before them 211.5 ->
+// 126.5 (as two key groups; 64.2 and 222.1 with one); 2048 124.0 -> 120.3 and at 6144
+// 447.7 -> 426.5; 37 at 4000 89.4 -> 87.4.  Running P V of the tile before beside the
+// softmax gave 472 for the 448.
 constexpr int kPreTile = 32;
 
 // 16-byte slot of K row `key` holding dims 8s .. 8s+7 (s ^ this): the 16 rows of one
@@ -852,7 +860,7 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
   // two V^T rows rather than sixteen).  A tile's 32 rows are contiguous from its first
   // row (one offset lookup per tile).
   typedef u32x4_t Pieces[2][PCH];  // a vector type: copies stay in registers
-  Pieces ra, rb;
+  Pieces ra;
   auto load_tile = [&](Pieces& r, int64_t t) {
     const int64_t off = p.kv.Row(b, g, t * TP);
     const uint32_t lim = static_cast<uint32_t>(min(last_row - t * TP, int64_t{TP - 1}));
@@ -920,10 +928,12 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
     bf16x8_t phi[CG], plo[CG];
 #pragma unroll
     for (int c = 0; c < CG; ++c) {
-      // lane (j, h), slot e = 4 tt + r: key 8h + e of query column j
+      // lane (j, h), slot e = 4 tt + r: key 8h + e of query column j (unscaled scores;
+      // the scale enters the exponent's fma, and a column without a live key subtracts 0,
+      // so -inf needs no test per score)
       float sc[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sc[e] = acc[c][e >> 2][e & 3] * p.scale;
+      for (int e = 0; e < 8; ++e) sc[e] = acc[c][e >> 2][e & 3];
       if (!full) {
         const int32_t lim = static_cast<int32_t>(min(qpos[c], kend - 1));  // keys <= lim are live
 #pragma unroll
@@ -935,7 +945,7 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
       for (int e = 1; e < 8; ++e) bm = fmaxf(bm, sc[e]);
       bm = fmaxf(bm, xor_partner<16>(bm, lane));
       bm = fmaxf(bm, xor_partner<32>(bm, lane));
-      const float mn = fmaxf(m_run[c], bm);
+      const float mn = fmaxf(m_run[c], bm * p.scale);
       // Rescale only when some column's maximum grew (multiplying by exp2(0) = 1 is
       // exact, so skipping it changes nothing); after the first tiles this is rare.
       if (__builtin_amdgcn_ballot_w64(mn > m_run[c]) != 0) {
@@ -949,15 +959,23 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
         }
       }
       m_run[c] = mn;
+      const float sub = mn == -INFINITY ? 0.0f : -mn;
       float sum = 0.0f;
+      uint32_t wh[4], wl[4];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = sc[e] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(sc[e] - mn);
-        sum += v;
-        const __bf16 hb = static_cast<__bf16>(v);
-        phi[c][e] = hb;
-        plo[c][e] = static_cast<__bf16>(v - static_cast<float>(hb));
+      for (int e = 0; e < 8; e += 2) {
+        typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+        const float v0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[e], p.scale, sub));
+        const float v1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[e + 1], p.scale, sub));
+        sum += v0;
+        sum += v1;
+        const uint32_t hp = __builtin_bit_cast(uint32_t, bf16x2_t{static_cast<__bf16>(v0), static_cast<__bf16>(v1)});
+        const float r0 = v0 - __uint_as_float(hp << 16), r1 = v1 - __uint_as_float(hp & 0xFFFF0000u);
+        wh[e / 2] = hp;
+        wl[e / 2] = __builtin_bit_cast(uint32_t, bf16x2_t{static_cast<__bf16>(r0), static_cast<__bf16>(r1)});
       }
+      phi[c] = __builtin_bit_cast(bf16x8_t, make_uint4(wh[0], wh[1], wh[2], wh[3]));
+      plo[c] = __builtin_bit_cast(bf16x8_t, make_uint4(wl[0], wl[1], wl[2], wl[3]));
       l_run[c] += sum;
     }
 #pragma unroll
@@ -973,89 +991,65 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
     }
   };
 
-  if constexpr (KS == 1) {
-    // tile t: in LDS buffer t & 1; its registers were loaded two iterations earlier
-    load_tile(ra, 0);
-    if (ntiles > 1) load_tile(rb, 1);
+  // The group's u-th tile is tile u KS + kg, in LDS buffer u & 1; the next one's registers
+  // are loaded before the tile is computed and stored after it.  Every group runs the
+  // loop of the group with the most tiles (the first), so all threads meet at the same
+  // barriers.  (Two register sets and a loop unrolled by two made the compiler move the
+  // running output between two sets of registers in every tile.)
+  const int64_t nu = (ntiles + KS - 1) / KS;                            // group 0's tiles
+  const int64_t nmine = ntiles > kg ? (ntiles - kg + KS - 1) / KS : 0;  // this group's
+  auto gt = [&](int64_t u) { return u * KS + kg; };
+  if (nmine > 0) {
+    load_tile(ra, gt(0));
     store_tile(ra, 0);
+  }
+  __syncthreads();
+  for (int64_t u = 0; u < nu; ++u) {
+    const int buf = static_cast<int>(u & 1);
+    if (u + 1 < nmine) load_tile(ra, gt(u + 1));
+    if (KS == 1 || u < nmine) compute(buf, gt(u));
+    if (u + 1 < nmine) store_tile(ra, buf ^ 1);
     __syncthreads();
-    int64_t t = 0;
-    for (; t + 1 < ntiles; t += 2) {
-      // even tile t in buffer 0; rb holds tile t + 1
-      if (t + 2 < ntiles) load_tile(ra, t + 2);
-      compute(0, t);
-      store_tile(rb, 1);
-      __syncthreads();
-      if (t + 3 < ntiles) load_tile(rb, t + 3);
-      compute(1, t + 1);
-      if (t + 2 < ntiles) store_tile(ra, 0);
-      __syncthreads();
-    }
-    if (t < ntiles) compute(0, t);
-  } else {
-    // The group's u-th tile is tile u KS + kg, in LDS buffer u & 1, loaded as above.
-    // Every group runs the loop of the group with the most tiles (the first), so all
-    // threads meet at the same barriers.
-    const int64_t nu = (ntiles + KS - 1) / KS;                            // group 0's tiles
-    const int64_t nmine = ntiles > kg ? (ntiles - kg + KS - 1) / KS : 0;  // this group's
-    auto gt = [&](int64_t u) { return u * KS + kg; };
-    if (nmine > 0) load_tile(ra, gt(0));
-    if (nmine > 1) load_tile(rb, gt(1));
-    if (nmine > 0) store_tile(ra, 0);
-    __syncthreads();
-    int64_t u = 0;
-    for (; u + 1 < nu; u += 2) {
-      if (u + 2 < nmine) load_tile(ra, gt(u + 2));
-      if (u < nmine) compute(0, gt(u));
-      if (u + 1 < nmine) store_tile(rb, 1);
-      __syncthreads();
-      if (u + 3 < nmine) load_tile(rb, gt(u + 3));
-      if (u + 1 < nmine) compute(1, gt(u + 1));
-      if (u + 2 < nmine) store_tile(ra, 0);
-      __syncthreads();
-    }
-    if (u < nmine) compute(0, gt(u));
   }
 
   if constexpr (KS == 2) {
-    // the second group's states into LDS (lane-contiguous words per wave: o in the K
-    // buffers, m and l in the V buffers), merged into the first group's on the same lanes
-    constexpr int OW = CG * DT * 4;  // o words per lane
-    static_assert(NW * OW * 64 * 4 <= static_cast<int>(sizeof(sk_)) &&
-                      NW * 2 * CG * 64 * 4 <= static_cast<int>(sizeof(sv_)),
+    // the second group's states into LDS, one column group at a time (lane-contiguous
+    // words per wave: o in the K buffers, m and l in the V buffers), merged into the first
+    // group's on the same lanes
+    constexpr int OW = DT * 4;  // o words per lane and column group
+    static_assert(NW * OW * 64 * 4 <= static_cast<int>(sizeof(sk_)) && NW * 2 * 64 * 4 <= static_cast<int>(sizeof(sv_)),
                   "merge records fit the tile buffers");
     float* reco = reinterpret_cast<float*>(&sk_[0][0][0]) + wave * OW * 64 + lane;
-    float* recm = reinterpret_cast<float*>(&sv_[0][0][0]) + wave * 2 * CG * 64 + lane;
-    __syncthreads();  // every group is done with its tiles
-    if (kg == 1) {
-#pragma unroll
-      for (int c = 0; c < CG; ++c) {
-        recm[(2 * c) * 64] = m_run[c];
-        recm[(2 * c + 1) * 64] = l_run[c];
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) reco[((c * DT + dt) * 4 + r) * 64] = o[c][dt][r];
-      }
-    }
-    __syncthreads();
-    if (kg == 1) return;
+    float* recm = reinterpret_cast<float*>(&sv_[0][0][0]) + wave * 2 * 64 + lane;
 #pragma unroll
     for (int c = 0; c < CG; ++c) {
-      // column j's scale factors (every lane of the column holds its maximum)
-      const float m2 = recm[(2 * c) * 64], l2 = recm[(2 * c + 1) * 64];
-      const float mn = fmaxf(m_run[c], m2);
-      const float f1 = m_run[c] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run[c] - mn);
-      const float f2 = m2 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m2 - mn);
-      l_run[c] = l_run[c] * f1 + l2 * f2;
-      m_run[c] = mn;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        // o[..][r] is column 4h + r: that column's factors
-        const float c1 = __shfl(f1, 16 * h + 4 * h + r), c2 = __shfl(f2, 16 * h + 4 * h + r);
+      __syncthreads();  // every group is done with its tiles, or with the records before
+      if (kg == 1) {
+        recm[0] = m_run[c];
+        recm[64] = l_run[c];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
-          o[c][dt][r] = o[c][dt][r] * c1 + reco[((c * DT + dt) * 4 + r) * 64] * c2;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) reco[(dt * 4 + r) * 64] = o[c][dt][r];
+      }
+      __syncthreads();
+      if (kg == 1) {
+        if (c == CG - 1) return;
+      } else {
+        // column j's scale factors (every lane of the column holds its maximum)
+        const float m2 = recm[0], l2 = recm[64];
+        const float mn = fmaxf(m_run[c], m2);
+        const float f1 = m_run[c] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run[c] - mn);
+        const float f2 = m2 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m2 - mn);
+        l_run[c] = l_run[c] * f1 + l2 * f2;
+        m_run[c] = mn;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          // o[..][r] is column 4h + r: that column's factors
+          const float c1 = __shfl(f1, 16 * h + 4 * h + r), c2 = __shfl(f2, 16 * h + 4 * h + r);
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) o[c][dt][r] = o[c][dt][r] * c1 + reco[(dt * 4 + r) * 64] * c2;
+        }
       }
     }
   }
@@ -1097,17 +1091,16 @@ void LaunchTimed(K kernel, dim3 grid, dim3 block, hipStream_t s, const AttnArgs&
 template <int D, int G, int CG, int NW, int KS>
 void LaunchPrefillShape(int64_t blocks, const AttnArgs& a, hipStream_t s) {
   constexpr int QB = NW * CG * (16 / G);
-  if constexpr (KS == 1)
-    RecordLaunch(blocks, NW * 64, 0, "attention_prefill<d=%d,g=%d,qb=%d>", D, G, QB);
-  else
-    RecordLaunch(blocks, NW * 64 * KS, 0, "attention_prefill<d=%d,g=%d,qb=%d,ks=%d>", D, G, QB, KS);
+  // (ks names the narrow shape; the threads per block tell the key groups of the others)
+  RecordLaunch(blocks, NW * 64 * KS, 0,
+               CG == 1 ? "attention_prefill<d=%d,g=%d,qb=%d,ks=%d>" : "attention_prefill<d=%d,g=%d,qb=%d>", D, G, QB, KS);
   LaunchTimed(attention_prefill_kernel<D, G, CG, NW, KS>, dim3(static_cast<unsigned>(blocks)), dim3(NW * 64 * KS), s,
               a);
 }
 
 // Query positions per block: the largest of 16/G x {4, 8, 16} that still gives every CU
-// a block (fewer re-reads of K/V per query), else the smallest, as two key groups of
-// four waves.
+// a block (fewer re-reads of K/V per query), else the smallest; the shapes of four query
+// waves as two key groups.
 template <int D, int G>
 void LaunchPrefillG(const AttnArgs& a, int64_t batch, hipStream_t s) {
   const int64_t per = a.hkv * batch, cus = DeviceCUs();
@@ -1117,7 +1110,7 @@ void LaunchPrefillG(const AttnArgs& a, int64_t batch, hipStream_t s) {
   if (D == 128 && blocks(16 * QT) >= cus)
     LaunchPrefillShape<D, G, 2, D == 128 ? 8 : 4, 1>(blocks(16 * QT), a, s);
   else if (blocks(8 * QT) >= cus)
-    LaunchPrefillShape<D, G, 2, 4, 1>(blocks(8 * QT), a, s);
+    LaunchPrefillShape<D, G, 2, 4, 2>(blocks(8 * QT), a, s);
   else
     LaunchPrefillShape<D, G, 1, 4, 2>(blocks(4 * QT), a, s);
 }

@@ -203,3 +203,30 @@ def test_batched_rows_past_lds(m, n, k, fmt):
     L.call("am_gfx950_linear", N.LinearArgs(p(xd), N.AM_DT_BF16, m, dw, p(out), N.AM_DT_F32, None, 3), stream())
     assert (np.abs(host(out) - ref) <= sums + 1e-30).all()
     del keep
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("start", [0, 31])
+def test_attention_prefill_two_key_groups(d, start):
+    """The middle prefill shape, two key groups merged one column group at a time: blocks
+    whose second group has no tile (the first positions), one tile less than the first, or
+    as many, a ragged last block, and columns that see no key of a group."""
+    hq, hkv, B, qb = 16, 4, 1, 32
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    S = (-(-cus // hkv) - 1) * qb + 5  # exactly enough blocks, the last of 5 positions
+    cap = start + S + 3
+    rng = np.random.default_rng(710 + d + start)
+    q = rbf(rng.standard_normal((S, hq * d), dtype=np.float32))
+    kc = rbf(rng.standard_normal((hkv, cap, d), dtype=np.float32))
+    vc = rbf(rng.standard_normal((hkv, cap, d), dtype=np.float32))
+    qd, kd, vd = (bf16_dev(bf16_rne_bits(x)) for x in (q, kc, vc))
+    out = empty((S, hq * d), torch.int16)
+    a = N.AttentionArgs(p(qd), p(kd), p(vd), p(out), S, hq, hkv, d, cap, start, None, 1, 0, 1, 0, None, 0)
+    L.call("am_gfx950_attention", a, stream())
+    assert launched() == f"attention_prefill<d={d},g=4,qb={qb}>"
+    got = O.bf16_to_f32(host(out).view(np.uint16)).reshape(S, hq * d)
+    for s in (0, 1, 4, 30, 31, 32, 33, 63, 64, 65, 95, 96, S - 6, S - 5, S - 1):
+        ref = O.attention(np.ascontiguousarray(q[s:s + 1]), kc, vc, 1, hq, hkv, d, cap, start + s)[0]
+        # P is held as bf16 hi + lo (2^-16 of a weight), the result rounded to bf16 (2^-9)
+        bad = np.abs(got[s] - ref) > 2.0 ** -8 * np.abs(ref) + 1e-4 * np.abs(ref).max()
+        assert not bad.any(), (s, np.argwhere(bad)[:8])
