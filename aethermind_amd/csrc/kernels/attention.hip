@@ -780,7 +780,27 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(AttnArgs p) {
 // 126.5 (as two key groups; 64.2 and 222.1 with one); 2048 124.0 -> 120.3 and at 6144
 // 447.7 -> 426.5; 37 at 4000 89.4 -> 87.4.  Running P V of the tile before beside the
 // softmax gave 472 for the 448.
+// The narrow shape (CG = 1) also splits the keys over blocks: a few dozen rows are 24 blocks
+// of 8 kv heads, which walk a long context tile after tile on a tenth of the CUs.  Grid
+// (blocks, splits); split i takes the i-th contiguous part of the block's tiles, writes its
+// columns' state as fp32 records (device-coherent, as the decode kernel's), and the block's
+// last split to finish merges all of them in split order.  A block's ticket is one byte, so
+// that every ticket lies in the workspace's first 256 bytes, which each user of a shared
+// workspace keeps zero between calls.  Whole INT4 8B layers, unsplit -> split (us): 16 rows
+// at 6000 keys 226 -> 125, 37 at 4000 190 -> 128, 100 at 3000 205 -> 165, 200 at 5000 307 ->
+// 260, 37 at 600 122.7 -> 118.6, 64 at 400 124.2 -> 121.8.  Launches that cannot reach
+// kPreSplitKeys run the kernel without the split's code (16 rows at 200: 110.3, with it
+// 111.2; at 300, two splits, 111.9 against 112.3).
 constexpr int kPreTile = 32;
+constexpr int kPreMaxSplits = 16;
+constexpr int64_t kPreMinKeys = 128;  // fewest keys of a split
+constexpr int64_t kPreSplitKeys = 512;  // launches that cannot reach as many keys run unsplit
+constexpr int64_t kMaxRows = 65535;   // query rows of a call
+
+// Bytes of one split's records of one block: 4 waves, per lane D / 4 output words, m and l.
+constexpr int64_t PreRecordBytes(int64_t d) { return 4 * (d / 4 + 2) * 64 * 4; }
+// The records start past the tickets of any call with these kv heads.
+int64_t PreRecordsAt(int64_t hkv) { return 256 * CeilDiv(kMaxRows * hkv * 4, 256); }
 
 // 16-byte slot of K row `key` holding dims 8s .. 8s+7 (s ^ this): the 16 rows of one
 // score MFMA operand fall into 16 distinct slots.
@@ -794,7 +814,7 @@ __device__ __forceinline__ int kswz(int key) {
 // 16-byte slot of V^T row d holding keys 8s .. 8s+7 (s ^ this)
 __device__ __forceinline__ int vswz(int d) { return (d >> 2) & 3; }
 
-template <int D, int G, int CG, int NW, int KS>
+template <int D, int G, int CG, int NW, int KS, bool SPLIT>
 __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArgs p) {
   static_assert(KS == 1 || KS == 2, "one or two key groups");
   constexpr int NT = NW * 64;                // threads of one key group
@@ -830,8 +850,7 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
   const int64_t s_last = s0 + QB - 1 < p.seq - 1 ? s0 + QB - 1 : p.seq - 1;
   int64_t kend = start + s_last + 1;  // keys the block needs: [0, kend)
   if (kend > p.cap) kend = p.cap;
-  const int64_t ntiles = (kend + TP - 1) / TP;
-
+  int64_t ntiles = (kend + TP - 1) / TP;
   // column group c of this wave: positions s0 + (wave * CG + c) * QT + j / G; its score
   // B operand (query column j at d = 32 kk + 8 h .. +8; zero for missing queries)
   int64_t qpos[CG];
@@ -846,9 +865,24 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
       uint4 v = *reinterpret_cast<const uint4*>(qp + 32 * kk);
-      if (qpos[c] < 0) v = make_uint4(0, 0, 0, 0);
+      if (s >= p.seq) v = make_uint4(0, 0, 0, 0);
       qop[c][kk] = __builtin_bit_cast(bf16x8_t, v);
     }
+  }
+  // This split's tiles [t0, t0 + ntiles) of the block's (after the query loads, which need
+  // no position; 32-bit divisions: the capacity is below 2^31).
+  int64_t t0 = 0;
+  int nsplit = 1;
+  if constexpr (SPLIT) {
+    if (kend >= 2 * kPreMinKeys) {
+      const uint32_t nt = static_cast<uint32_t>(ntiles);
+      const uint32_t ns = min(static_cast<uint32_t>(kend / kPreMinKeys), static_cast<uint32_t>(p.splits));
+      const uint32_t per = (nt + ns - 1) / ns;
+      nsplit = static_cast<int>((nt + per - 1) / per);
+      t0 = blockIdx.y * per;
+      ntiles = min(ntiles - t0, static_cast<int64_t>(per));
+    }
+    if (static_cast<int>(blockIdx.y) >= nsplit) return;  // surplus block for this context
   }
   const uint16_t* kc0 = static_cast<const uint16_t*>(p.kc);
   const uint16_t* vc0 = static_cast<const uint16_t*>(p.vc);
@@ -998,7 +1032,7 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
   // running output between two sets of registers in every tile.)
   const int64_t nu = (ntiles + KS - 1) / KS;                            // group 0's tiles
   const int64_t nmine = ntiles > kg ? (ntiles - kg + KS - 1) / KS : 0;  // this group's
-  auto gt = [&](int64_t u) { return u * KS + kg; };
+  auto gt = [&](int64_t u) { return t0 + u * KS + kg; };
   if (nmine > 0) {
     load_tile(ra, gt(0));
     store_tile(ra, 0);
@@ -1034,7 +1068,7 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
       }
       __syncthreads();
       if (kg == 1) {
-        if (c == CG - 1) return;
+        if (c == CG - 1 && nsplit == 1) return;
       } else {
         // column j's scale factors (every lane of the column holds its maximum)
         const float m2 = recm[0], l2 = recm[64];
@@ -1051,6 +1085,97 @@ __global__ __launch_bounds__(NW * 64 * KS) void attention_prefill_kernel(AttnArg
           for (int dt = 0; dt < DT; ++dt) o[c][dt][r] = o[c][dt][r] * c1 + reco[(dt * 4 + r) * 64] * c2;
         }
       }
+    }
+  }
+
+  if constexpr (SPLIT) {
+    static_assert(CG == 1 && NW == 4 && KS == 2 && DT % 2 == 0, "the records' layout, and two groups to merge them");
+    if (nsplit > 1) {
+      constexpr int kWaveBytes = (DT * 4 + 2) * 64 * 4, kMl = DT * 64 * 16;
+      auto region = [&](int sp) {
+        uint8_t* at = reinterpret_cast<uint8_t*>(p.part) +
+                      ((static_cast<int64_t>(blockIdx.x) * p.splits + sp) * NW + wave) * kWaveBytes;
+        return __builtin_amdgcn_make_buffer_rsrc(at, 0, kWaveBytes, kRawBufferFlags);
+      };
+      if (kg == 0) {
+        const __amdgpu_buffer_rsrc_t mine = region(static_cast<int>(blockIdx.y));
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o[0][dt]), mine, (dt * 64 + lane) * 16, 0,
+                                                 kCpolSc1);
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{__float_as_uint(m_run[0]), __float_as_uint(l_run[0])}, mine,
+                                              kMl + lane * 8, 0, kCpolSc1);
+        __builtin_amdgcn_s_waitcnt(0);  // acknowledged before the ticket
+      }
+      __syncthreads();
+      int* last = reinterpret_cast<int*>(&sv_[0][0][0]);  // the groups' records there are consumed
+      if (threadIdx.x == 0) {
+        const int sh = 8 * (blockIdx.x & 3);
+        unsigned* tk = p.tickets + (blockIdx.x >> 2);
+        const unsigned old = __hip_atomic_fetch_add(tk, 1u << sh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool end = ((old >> sh) & 255u) == static_cast<unsigned>(nsplit - 1);
+        *last = end;
+        if (end)
+          __hip_atomic_fetch_sub(tk, static_cast<unsigned>(nsplit) << sh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
+      if (*last == 0) return;
+      // Merge: the two key groups take half of the output tiles each.  Records past the
+      // last split are read as the last one and left out.
+      constexpr int HD = DT / 2;
+      float ms[kPreMaxSplits], f[kPreMaxSplits], ls[kPreMaxSplits];
+      float mx = -INFINITY, lr = 0.0f;
+#pragma unroll
+      for (int sp = 0; sp < kPreMaxSplits; ++sp) {
+        const u32x2_t w = __builtin_amdgcn_raw_buffer_load_b64(region(min(sp, nsplit - 1)), kMl + lane * 8, 0, kCpolSc1);
+        ms[sp] = __uint_as_float(w[0]);
+        ls[sp] = __uint_as_float(w[1]);
+      }
+#pragma unroll
+      for (int sp = 0; sp < kPreMaxSplits; ++sp) mx = fmaxf(mx, ms[sp]);
+#pragma unroll
+      for (int sp = 0; sp < kPreMaxSplits; ++sp) {
+        f[sp] = ms[sp] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms[sp] - mx);
+        if (sp < nsplit) lr += ls[sp] * f[sp];
+      }
+      f32x4_t sum[HD];
+#pragma unroll
+      for (int i = 0; i < HD; ++i) sum[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s4 = 0; s4 < kPreMaxSplits; s4 += 4) {
+        if (s4 >= nsplit) break;
+        u32x4_t v[4][HD];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const __amdgpu_buffer_rsrc_t rec = region(min(s4 + e, nsplit - 1));
+#pragma unroll
+          for (int i = 0; i < HD; ++i)
+            v[e][i] = __builtin_amdgcn_raw_buffer_load_b128(rec, ((kg * HD + i) * 64 + lane) * 16, 0, kCpolSc1);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (s4 + e >= nsplit) break;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float fr = __shfl(f[s4 + e], 16 * h + 4 * h + r);  // column 4h + r's
+#pragma unroll
+            for (int i = 0; i < HD; ++i) sum[i][r] += __uint_as_float(v[e][i][r]) * fr;
+          }
+        }
+      }
+      lr += xor_partner<16>(lr, lane);
+      lr += xor_partner<32>(lr, lane);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int q = 4 * h + r;
+        const float lq = __shfl(lr, 16 * h + q);
+        const int64_t sq = s0 + wave * QT + q / G;
+        if (sq >= p.seq) continue;
+        uint16_t* out = static_cast<uint16_t*>(p.out) + ((b * p.seq + sq) * p.hq + g * G + q % G) * D + kg * HD * 16;
+#pragma unroll
+        for (int i = 0; i < HD; ++i) out[16 * i + j] = f32_to_bf16_bits(lq > 0.0f ? sum[i][r] / lq : 0.0f);
+      }
+      return;
     }
   }
 
@@ -1088,21 +1213,24 @@ void LaunchTimed(K kernel, dim3 grid, dim3 block, hipStream_t s, const AttnArgs&
   }
 }
 
-template <int D, int G, int CG, int NW, int KS>
+template <int D, int G, int CG, int NW, int KS, bool SPLIT = false>
 void LaunchPrefillShape(int64_t blocks, const AttnArgs& a, hipStream_t s) {
   constexpr int QB = NW * CG * (16 / G);
   // (ks names the narrow shape; the threads per block tell the key groups of the others)
-  RecordLaunch(blocks, NW * 64 * KS, 0,
-               CG == 1 ? "attention_prefill<d=%d,g=%d,qb=%d,ks=%d>" : "attention_prefill<d=%d,g=%d,qb=%d>", D, G, QB, KS);
-  LaunchTimed(attention_prefill_kernel<D, G, CG, NW, KS>, dim3(static_cast<unsigned>(blocks)), dim3(NW * 64 * KS), s,
-              a);
+  const char* name = CG > 1          ? "attention_prefill<d=%d,g=%d,qb=%d>"
+                     : !SPLIT        ? "attention_prefill<d=%d,g=%d,qb=%d,ks=%d>"
+                                     : "attention_prefill<d=%d,g=%d,qb=%d,ks=%d,splits=%d>";
+  const dim3 grid(static_cast<unsigned>(blocks), SPLIT ? static_cast<unsigned>(a.splits) : 1u);
+  RecordLaunch(GridBlocks(grid), NW * 64 * KS, 0, name, D, G, QB, KS, a.splits);
+  LaunchTimed(attention_prefill_kernel<D, G, CG, NW, KS, SPLIT>, grid, dim3(NW * 64 * KS), s, a);
 }
 
 // Query positions per block: the largest of 16/G x {4, 8, 16} that still gives every CU
 // a block (fewer re-reads of K/V per query), else the smallest; the shapes of four query
-// waves as two key groups.
+// waves as two key groups.  The smallest splits its keys as far as the blocks stay within
+// one round, a split has kPreMinKeys keys and the workspace (of ws_bytes) holds the records.
 template <int D, int G>
-void LaunchPrefillG(const AttnArgs& a, int64_t batch, hipStream_t s) {
+void LaunchPrefillG(AttnArgs a, int64_t batch, int64_t ws_bytes, hipStream_t s) {
   const int64_t per = a.hkv * batch, cus = DeviceCUs();
   auto blocks = [&](int64_t qb) { return CeilDiv(a.seq, qb) * per; };
   constexpr int QT = 16 / G;
@@ -1111,17 +1239,27 @@ void LaunchPrefillG(const AttnArgs& a, int64_t batch, hipStream_t s) {
     LaunchPrefillShape<D, G, 2, D == 128 ? 8 : 4, 1>(blocks(16 * QT), a, s);
   else if (blocks(8 * QT) >= cus)
     LaunchPrefillShape<D, G, 2, 4, 2>(blocks(8 * QT), a, s);
-  else
-    LaunchPrefillShape<D, G, 1, 4, 2>(blocks(4 * QT), a, s);
+  else {
+    const int64_t nb = blocks(4 * QT);
+    // (a device start position: the longest context is the capacity)
+    const int64_t keys = a.start_dev != nullptr ? a.cap : a.start + a.seq;
+    const int64_t ns = std::min<int64_t>(std::min<int64_t>(kPreMaxSplits, cus / nb), keys / kPreMinKeys);
+    if (a.part != nullptr && ns > 1 && keys >= kPreSplitKeys && nb <= 256 && PreRecordsAt(a.hkv) + nb * ns * PreRecordBytes(D) <= ws_bytes) {
+      a.splits = static_cast<int32_t>(ns);
+      LaunchPrefillShape<D, G, 1, 4, 2, true>(nb, a, s);
+    } else {
+      LaunchPrefillShape<D, G, 1, 4, 2>(nb, a, s);
+    }
+  }
 }
 
 template <int D>
-am_status_code LaunchPrefill(int64_t G, int64_t batch, const AttnArgs& a, hipStream_t s) {
+am_status_code LaunchPrefill(int64_t G, int64_t batch, const AttnArgs& a, int64_t ws_bytes, hipStream_t s) {
   switch (G) {
-    case 1: LaunchPrefillG<D, 1>(a, batch, s); break;
-    case 2: LaunchPrefillG<D, 2>(a, batch, s); break;
-    case 4: LaunchPrefillG<D, 4>(a, batch, s); break;
-    case 8: LaunchPrefillG<D, 8>(a, batch, s); break;
+    case 1: LaunchPrefillG<D, 1>(a, batch, ws_bytes, s); break;
+    case 2: LaunchPrefillG<D, 2>(a, batch, ws_bytes, s); break;
+    case 4: LaunchPrefillG<D, 4>(a, batch, ws_bytes, s); break;
+    case 8: LaunchPrefillG<D, 8>(a, batch, ws_bytes, s); break;
     default: return SetLastError(AM_STATUS_UNIMPLEMENTED, "attention: q heads per kv head must be 1, 2, 4 or 8");
   }
   AM_RETURN_IF_LAUNCH_FAILED("attention");
@@ -1135,6 +1273,15 @@ int ChooseSplits(int64_t seq, int64_t cap, int32_t requested) {
   if (s < 1) s = 1;
   if (s > kMaxSplits) s = kMaxSplits;
   return static_cast<int>(s);
+}
+
+// Workspace that a call needs.
+int64_t RequiredBytes(int64_t batch, int64_t seq, int64_t hq, int64_t hkv, int64_t head_dim, int64_t capacity,
+                      int32_t num_splits) {
+  const int splits = ChooseSplits(seq, capacity, num_splits);
+  if (splits == 1) return 0;
+  const int64_t tickets = 256 * CeilDiv(batch * seq * hkv * 4, 256);
+  return tickets + batch * seq * hq * splits * (head_dim + 4) * 4;
 }
 
 template <int D, int NW>
@@ -1179,10 +1326,12 @@ using namespace am;
 
 extern "C" int64_t am_gfx950_attention_workspace_bytes(int64_t batch, int64_t seq, int64_t hq, int64_t hkv,
                                                        int64_t head_dim, int64_t capacity, int32_t num_splits) {
-  const int splits = ChooseSplits(seq, capacity, num_splits);
-  if (splits == 1) return 0;
-  const int64_t tickets = 256 * CeilDiv(batch * seq * hkv * 4, 256);
-  return tickets + batch * seq * hq * splits * (head_dim + 4) * 4;
+  const int64_t need = RequiredBytes(batch, seq, hq, hkv, head_dim, capacity, num_splits);
+  // Prefill rows: what lets any number of rows up to this one split its keys (optional).
+  const int64_t cus = DeviceCUs();
+  if (seq > 1 && num_splits <= 0 && capacity >= kPreSplitKeys && 2 * hkv * std::max<int64_t>(batch, 1) <= cus)
+    return std::max(need, PreRecordsAt(hkv) + cus * PreRecordBytes(head_dim));
+  return need;
 }
 
 // ---- zero-allocation variant -----------------------------------------------------
@@ -1229,9 +1378,9 @@ extern "C" am_status_code am_gfx950_attention_noalloc(const am_gfx950_attention_
   AM_CHECK_ARG(a->hq > 0 && a->hkv > 0 && a->seq > 0 && a->capacity > 0 && a->head_dim > 0,
                "attention_noalloc: bad shape");
   const int64_t batch = a->batch > 0 ? a->batch : 1;
-  AM_CHECK_ARG(batch * a->seq <= 65535, "attention: too many query rows");
-  const int64_t need = am_gfx950_attention_workspace_bytes(batch, a->seq, a->hq, a->hkv, a->head_dim, a->capacity,
-                                                           a->num_splits);
+  AM_CHECK_ARG(batch * a->seq <= kMaxRows, "attention: too many query rows");
+  // (prefill rows run unsplit here, without the scratch)
+  const int64_t need = RequiredBytes(batch, a->seq, a->hq, a->hkv, a->head_dim, a->capacity, a->num_splits);
   if (need > kNoAllocScratchBytes) {
     char msg[160];
     std::snprintf(msg, sizeof(msg), "attention_noalloc: needs %lld bytes of split scratch, the maximum is %lld",
@@ -1266,14 +1415,13 @@ extern "C" am_status_code am_gfx950_attention(const am_gfx950_attention_args* a,
   AM_CHECK_ARG(a->head_dim == 64 || a->head_dim == 128, "attention: head_dim must be 64 or 128");
   AM_CHECK_ARG(a->seq > 0 && a->capacity > 0, "attention: bad shape");
   const int64_t batch = a->batch > 0 ? a->batch : 1;
-  AM_CHECK_ARG(batch * a->seq <= 65535, "attention: too many query rows");
+  AM_CHECK_ARG(batch * a->seq <= kMaxRows, "attention: too many query rows");
   AM_CHECK_ARG(a->q && a->k_cache && a->v_cache && a->out, "attention: null pointer");
   if (a->start_pos_dev == nullptr)
     AM_CHECK_ARG(a->start_pos >= 0 && a->start_pos + a->seq <= a->capacity, "KV read exceeds committed token range");
   const int splits = ChooseSplits(a->seq, a->capacity, a->num_splits);
   AM_CHECK_ARG(splits >= 1 && splits <= 1024, "attention: bad split count");
-  const int64_t need = am_gfx950_attention_workspace_bytes(batch, a->seq, a->hq, a->hkv, a->head_dim, a->capacity,
-                                                           a->num_splits);
+  const int64_t need = RequiredBytes(batch, a->seq, a->hq, a->hkv, a->head_dim, a->capacity, a->num_splits);
   if (splits > 1) AM_CHECK_ARG(a->workspace != nullptr && a->workspace_bytes >= need, "attention: workspace too small");
   AttnArgs p{};
   p.q = a->q;
@@ -1330,7 +1478,16 @@ extern "C" am_status_code am_gfx950_attention(const am_gfx950_attention_args* a,
   if (a->dtype == AM_DT_BF16) {
     // prefill: MFMA kernel, one block per (16 query columns per wave) x kv head x row
     AM_CHECK_ARG(a->capacity * a->head_dim < (int64_t{1} << 31), "attention: cache too large for 32-bit offsets");
-    return a->head_dim == 128 ? LaunchPrefill<128>(G, batch, p, s) : LaunchPrefill<64>(G, batch, p, s);
+    // and split of the keys where a workspace allows it
+    p.splits = 1;
+    p.part = nullptr;
+    if (a->num_splits <= 0 && a->workspace != nullptr && (reinterpret_cast<uintptr_t>(a->workspace) & 15u) == 0) {
+      uint8_t* ws = static_cast<uint8_t*>(a->workspace);
+      p.tickets = reinterpret_cast<unsigned*>(ws);
+      p.part = reinterpret_cast<float*>(ws + PreRecordsAt(a->hkv));
+    }
+    return a->head_dim == 128 ? LaunchPrefill<128>(G, batch, p, a->workspace_bytes, s)
+                              : LaunchPrefill<64>(G, batch, p, a->workspace_bytes, s);
   }
   // fp32 activations: the VALU kernel
   const dim3 grid(static_cast<unsigned>(splits), static_cast<unsigned>(a->hkv), static_cast<unsigned>(batch * a->seq));

@@ -252,7 +252,9 @@ am_status_code am_gfx950_kv_update(const am_gfx950_kv_update_args* args, void* h
  * no split is possible), whose first 4*hkv*batch*seq bytes (split tickets) must be
  * zero before the first call; the kernel leaves them zero.  Decode rows are split
  * over positions when the context is long; the last block of each (row, kv head)
- * merges the partial records, so one launch produces the output.
+ * merges the partial records, so one launch produces the output.  Few bf16 prefill rows
+ * (seq > 1) over a long context are split the same way when the workspace is given; it is
+ * optional there, and the bytes reported cover every smaller seq.
  * batch > 1 stacks independent sequences: q [batch][seq][hq*d], caches
  * [batch] planes of cache_batch_stride elements, start positions start_pos_dev[b].
  * pages != NULL (bf16 only): paged caches, sequence b's table row b. */
@@ -281,9 +283,9 @@ int64_t am_gfx950_attention_workspace_bytes(int64_t batch, int64_t seq, int64_t 
  * am_gfx950_attention_noalloc_max_bytes() bytes (8 MiB) that each device holds until
  * the process ends.  No counterpart in the reference: it is for callers that cannot
  * allocate (code under HIP graph capture, serving loops that forbid hipMalloc).
- * args->workspace must be NULL and args->workspace_bytes 0; a shape whose
+ * args->workspace must be NULL and args->workspace_bytes 0; a decode shape whose
  * am_gfx950_attention_workspace_bytes exceeds the maximum is rejected with
- * AM_STATUS_RESOURCE_EXHAUSTED.  Each call clears its tickets with a kernel on
+ * AM_STATUS_RESOURCE_EXHAUSTED, and automatic prefill runs unsplit.  Each call clears its tickets with a kernel on
  * hip_stream (no memset), then launches the same kernels as am_gfx950_attention.
  * Every call on one device shares that device's array: calls that overlap on one
  * device (different streams, concurrently) race and must not be issued. */

@@ -230,3 +230,51 @@ def test_attention_prefill_two_key_groups(d, start):
         # P is held as bf16 hi + lo (2^-16 of a weight), the result rounded to bf16 (2^-9)
         bad = np.abs(got[s] - ref) > 2.0 ** -8 * np.abs(ref) + 1e-4 * np.abs(ref).max()
         assert not bad.any(), (s, np.argwhere(bad)[:8])
+
+
+@pytest.mark.parametrize("m,B,starts", [(2, 1, [4094]), (17, 2, [0, 3000]), (37, 1, [600]), (37, 2, [218, 219]), (128, 1, [4000]), (130, 1, [255])])
+@pytest.mark.parametrize("d,g", [(128, 4), (64, 8)])
+@pytest.mark.parametrize("paged", [False, True])
+def test_attention_prefill_split_keys(m, B, starts, d, g, paged):
+    """Few prefill rows over a long context, the keys split over blocks: contexts below and
+    at two splits' keys, surplus blocks, splits whose keys some columns do not see, ragged
+    query blocks, two sequences; against fp64 attention.  The workspace serves a batched
+    decode call between two prefill calls, and every ticket is zero after each."""
+    hkv, cap = 4, 4608
+    hq, gen = g * hkv, torch.Generator("cuda").manual_seed(m + B)
+    k, v = (torch.randn((B, hkv, cap, d), device="cuda", generator=gen).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn((B, m, hq * d), device="cuda", generator=gen).to(torch.bfloat16)
+    kd, vd, pages = k, v, None
+    if paged:
+        per = cap // 64
+        table = torch.from_numpy(np.random.default_rng(m).permutation(B * per).astype(np.int32)).cuda().view(B, per)
+        kd, vd = (torch.empty((B * per, hkv, 64, d), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        for src, dst in ((k, kd), (v, vd)):
+            dst[table.long().view(-1)] = src.view(B, hkv, per, 64, d).transpose(1, 2).reshape(B * per, hkv, 64, d)
+        pages = C.pointer(N.KvPages(p(table), 64, per, B * per, None))
+    posd = dev(np.array(starts, np.int64))
+    wsb = max(L.am_gfx950_attention_workspace_bytes(B, s, hq, hkv, d, cap, 0) for s in (1, m))
+    assert L.am_gfx950_attention_workspace_bytes(B, m, hq, hkv, d, cap, 0) >= L.am_gfx950_attention_workspace_bytes(B, 2, hq, hkv, d, cap, 0)
+    ws = torch.zeros(wsb, dtype=torch.uint8, device="cuda")
+
+    def call(rows, qt, out):
+        L.call("am_gfx950_attention", N.AttentionArgs(p(qt), p(kd), p(vd), p(out), rows, hq, hkv, d, cap, 0, p(posd), B,
+                                                      hkv * cap * d, 1, 0, p(ws), wsb, pages), stream())
+        assert not bool(ws[:256].any())
+
+    outs = []
+    for _ in range(2):
+        outs.append(empty((B, m, hq, d), torch.bfloat16))
+        call(m, q, outs[-1])
+        assert f"ks=2,splits={min(16, torch.cuda.get_device_properties(0).multi_processor_count // (B * hkv * -(-m // (64 // g))))}>" in launched()
+        call(1, q, empty((B, hq, d), torch.bfloat16))
+    assert torch.equal(outs[0], outs[1])
+    for b in range(B):
+        for s in sorted({0, 1, m // 2, m - 1}):
+            n = starts[b] + s + 1
+            kr, vr = (t[b, :, :n].double().repeat_interleave(g, 0) for t in (k, v))
+            sc = (kr * q[b, s].double().view(hq, 1, d)).sum(-1) / d ** 0.5
+            ref = (torch.softmax(sc, -1).unsqueeze(-1) * vr).sum(1)
+            err = (outs[0][b, s].double() - ref).abs()
+            # a bf16 rounding of the output and P in bf16 hi + lo (2^-16 of the row's largest value)
+            assert bool((err <= ref.abs() * 2.0 ** -8 + 2.0 ** -15 * vr.abs().max()).all()), (b, s)
