@@ -217,11 +217,13 @@ __device__ __forceinline__ uint32_t nibble16(uint32_t v) {
   return d;
 }
 
+constexpr uint32_t kZeroCodes = 0x88888888u;  // 8 nibbles of q = 0
+
 // 8 nibbles q+8 in device tile order -> 8 bf16 values q / 16 (exact) in k order: the
 // nibbles of k 0, 4, 1, 5 are the low halves of bytes 0..3, those of k 2, 6, 3, 7 the
 // high halves.
 __device__ __forceinline__ bf16x8_t unpack8(uint32_t word) {
-  const uint32_t lo = word ^ 0x88888888u, hi = lo >> 4;
+  const uint32_t lo = word ^ kZeroCodes, hi = lo >> 4;
   const uint32_t d0 = __builtin_amdgcn_perm(nibble16<2>(lo), nibble16<0>(lo), 0x07060302u);
   const uint32_t d1 = __builtin_amdgcn_perm(nibble16<2>(hi), nibble16<0>(hi), 0x07060302u);
   const uint32_t d2 = __builtin_amdgcn_perm(nibble16<3>(lo), nibble16<1>(lo), 0x07060302u);
@@ -409,6 +411,7 @@ __global__ __launch_bounds__((Shape<WF, TILE>::kThreads), (Shape<WF, TILE>::BPC)
   RawB ob[NT];
   bf16x8_t bfr[2][NT];
   uint32_t sraw[NT];       // INT4: the group's scale dwords
+  bool dead = false;       // INT4: some lane's scale of the group is zero
   float sc[NT];            // INT4: the scale the sums are in units of
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
@@ -434,14 +437,18 @@ __global__ __launch_bounds__((Shape<WF, TILE>::kThreads), (Shape<WF, TILE>::BPC)
     for (int nt = 0; nt < NT; ++nt)
       sraw[nt] = *reinterpret_cast<const uint32_t*>(lds + soff + nt * 64 + (g & (S::kScSlots - 1)) * S::kScSlot);
   };
-  // A group begins: the sums so far change to its unit.  A zero scale counts as 2^-60:
-  // the codes the quantizer stores with it are 0, and others vanish beside any sum.
+  auto group_bits = [&](int32_t g, int nt) {
+    return ((shalf + g) & 1) ? (sraw[nt] >> 16) : (sraw[nt] & 0xFFFFu);
+  };
+  // A group begins: the sums so far change to its unit; a zero scale leaves them in theirs.
+  // (The smallest fp16 scale is 2^-24: sums below 2^108 stay finite in any unit.)
   auto open_group = [&](int32_t g, float (&ratio)[NT]) {
+    bool zero = false;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      const uint32_t bits = ((shalf + g) & 1) ? (sraw[nt] >> 16) : (sraw[nt] & 0xFFFFu);
-      float s = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(bits)));
-      if (s == 0.0f) s = 0x1p-60f;
+      float s = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(group_bits(g, nt))));
+      zero = zero || s == 0.0f;
+      if (s == 0.0f) s = sc[nt];
       // sc / s: reciprocal and one correction (not where that meets an infinity)
       const float inv = __builtin_amdgcn_rcpf(s);
       float q = sc[nt] * inv;
@@ -449,6 +456,27 @@ __global__ __launch_bounds__((Shape<WF, TILE>::kThreads), (Shape<WF, TILE>::BPC)
       if (e == e) q = __builtin_fmaf(e, inv, q);
       ratio[nt] = s == sc[nt] ? 1.0f : q;
       sc[nt] = s;
+    }
+    dead = __builtin_amdgcn_ballot_w64(zero) != 0;
+  };
+  // A group of zero scale adds nothing: its codes in step j become 0 (the quantizer stores
+  // 0 with such a scale, other packers may not), the first slice's in the registers they
+  // were converted to and the others in the LDS words that this lane reads.  The branch,
+  // which ordinary weights never take, costs up to 1% of a launch (512 x 28672 x 4096 133.8
+  // -> 135.3 us); masking every conversion cost 1-6%, and a zero scale taken as 2^-60 left
+  // sums of 1e-17 for rows of zero scales and overflowed above 5e21.
+  auto drop_zero_scale = [&](int32_t g, int32_t j) {
+    if constexpr (S::kI4) {
+      if (__builtin_expect(dead, 0)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          if ((group_bits(g, nt) & 0x7FFFu) == 0u) {
+            bfr[0][nt] = bf16x8_t{};
+#pragma unroll
+            for (int kk = 1; kk < KK; ++kk) *reinterpret_cast<uint32_t*>(lds + (j % NST) * STG + boff[nt][kk]) = kZeroCodes;
+          }
+        wait_lds();
+      }
     }
   };
   // MFMAs of slice kk; RESCALE: the first slice of an INT4 group.  As soon as a row of
@@ -523,9 +551,13 @@ __global__ __launch_bounds__((Shape<WF, TILE>::kThreads), (Shape<WF, TILE>::BPC)
   if constexpr (S::kI4) {
     for (int32_t g = g0; g < g1; ++g) {
       open_group(g, ratio);
+      drop_zero_scale(g, j);
       step(j, spg == 1 ? g + 1 : -1, std::true_type{}, ratio);
       ++j;
-      for (int32_t t = 1; t < spg; ++t, ++j) step(j, t + 1 == spg ? g + 1 : -1, std::false_type{}, ratio);
+      for (int32_t t = 1; t < spg; ++t, ++j) {
+        drop_zero_scale(g, j);
+        step(j, t + 1 == spg ? g + 1 : -1, std::false_type{}, ratio);
+      }
     }
   } else {
     for (; j < nk; ++j) step(j, -1, std::false_type{}, ratio);

@@ -111,29 +111,36 @@ def test_prefill_gemm_tiles(shape, fmt):
     del keep
 
 
-def test_prefill_gemm_zero_scale_groups():
-    """INT4 groups whose scale is zero but whose codes are not add nothing."""
-    m, n, k, group = 70, 256, 512, 128
+@pytest.mark.parametrize("m,n,k,group", [(70, 256, 512, 128), (300, 512, 512, 64), (257, 16392, 384, 128),
+                                         (1030, 12296, 512, 128)])
+@pytest.mark.parametrize("size", [1.0, 2.0 ** 80])
+def test_prefill_gemm_zero_scale_groups(m, n, k, group, size):
+    """INT4 groups whose scale is zero but whose codes are not add nothing, in each tile:
+    an output row of zero scales is exactly zero, and sums of any size stay what they were
+    before the group.  Bar as above."""
     rng = np.random.default_rng(5)
     codes = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
     sc = (rng.random((n, k // group), dtype=np.float32) * 0.1).astype(np.float16)
     sc[::2, 0] = 0
     sc[::3, 2] = 0
-    sc[5, :] = 0
+    sc[1::4, -1] = -0.0
+    sc[5::40, :] = 0
     logical, scales = dev(codes), dev(sc.view(np.int16))
     data = torch.zeros(n * k // 2, dtype=torch.uint8, device="cuda")
     dsc = torch.zeros(n * (k // group), dtype=torch.int16, device="cuda")
     dw = N.Weight(p(data), p(dsc), n, k, N.AM_WF_INT4, group)
     L.call("am_gfx950_pack_int4", N.PackInt4Args(p(logical), p(scales), dw), stream())
     q = np.stack([codes & 15, codes >> 4], -1).reshape(n, k).astype(np.int32)
-    w = np.where(q > 7, q - 16, q) * np.repeat(sc.astype(np.float64), group, 1)
-    x = act_rows(8, m, k)
-    xd = bf16_dev(bf16_rne_bits(x))
+    w = dev(np.where(q > 7, q - 16, q) * np.repeat(sc.astype(np.float64), group, 1))
+    x = act_rows(8, m, k) * np.float32(size)
+    xd, xt = bf16_dev(bf16_rne_bits(x)), dev(x).double()
     out = empty((m, n), torch.bfloat16)
     L.call("am_gfx950_linear", N.LinearArgs(p(xd), N.AM_DT_BF16, m, dw, p(out), N.AM_DT_BF16, None, 2), stream())
-    ref = x.astype(np.float64) @ w.T
-    bar = np.abs(ref) * 2.0 ** -8 + k * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + 1e-12
-    assert (np.abs(out.double().cpu().numpy() - ref) <= bar).all()
+    ref = xt @ w.T
+    bar = ref.abs() * 2.0 ** -8 + k * 2.0 ** -24 * (xt.abs() @ w.abs().T)
+    err = (out.double() - ref).abs()
+    assert bool((err <= bar).all()), (launched(), float((err - bar).max()))
+    assert not bool(out[:, 5::40].any())
 
 
 @pytest.mark.parametrize("B,hkv", [(16, 8), (12, 8), (9, 8), (5, 8), (64, 8), (24, 2)])
