@@ -9,12 +9,12 @@
 // to the MFMA's registers: a lane's 16-byte load of row (lane % 16), values 4 (lane / 16)
 // to + 3 of a chunk, is its operand of four MFMAs (MFMA e takes value e of every lane,
 // for X and W alike, so the chunk's 16 k values are summed in an order of their own).
-// The waves' partial tiles meet in LDS and are summed in wave order.
+// The waves' partial tiles meet in LDS and are summed in pairs.
 //   Tiles: 16 x 16 while 32 x 32 tiles would leave CUs without a block (48 x 512 x 512:
 //   96 blocks), 32 x 32 above (half the operand bytes per product).
 // It replaces one GEMV launch per row: the prefill of 48 rows through the 4-layer 512-wide
-// model took 1,344 launches of 2.5-3.3 us, now 28 of 5.0-6.5 us (a 48-token prompt and 32
-// greedy tokens 7.8 -> 3.8 ms).
+// model took 1,344 launches of 2.5-3.3 us, now 28 of 5.0-8.3 us (a 48-token prompt and 32
+// greedy tokens 7.8 -> 3.9 ms).
 
 #include "am_gemv_common.h"
 #include "am_launch_timing.h"
@@ -34,9 +34,11 @@ struct GemmF32Args {
   int32_t M, N, K, tiles_m;
 };
 
-// U: chunks of loads in flight per wave
+// U: chunks of loads in flight per wave (a power of two).  Two blocks per CU at least, which
+// keeps the MFMAs' results in registers that additions can read (without the bound they are
+// copied there: 48 x 512 x 1376 9.1 us).
 template <int MT, int NT, int U>
-__global__ __launch_bounds__(kWavesF * 64) void gemm_f32_kernel(GemmF32Args p) {
+__global__ __launch_bounds__(kWavesF * 64, 2) void gemm_f32_kernel(GemmF32Args p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int32_t tn = blockIdx.x / p.tiles_m, tm = blockIdx.x - tn * p.tiles_m;
@@ -55,16 +57,11 @@ __global__ __launch_bounds__(kWavesF * 64) void gemm_f32_kernel(GemmF32Args p) {
     const int32_t row = n0 + 16 * i + r;
     wr[i] = p.w + static_cast<int64_t>(row < p.N ? row : 0) * p.K;
   }
-  // one running sum per value of the 16-byte pieces: four independent MFMA chains, and
-  // sums of K / 64 products each before they meet (the error of one chain over a wave's
-  // whole share of K measured 1.4 times the GEMV's)
-  f32x4_t acc[4][MT][NT];
+  f32x4_t acc[MT][NT];
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) acc[e][i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   // chunk c holds k values 16 c .. 16 c + 15; K % 4 == 0, so a lane's four values are
   // all inside K or all past it (then zero on both sides)
@@ -92,6 +89,13 @@ __global__ __launch_bounds__(kWavesF * 64) void gemm_f32_kernel(GemmF32Args p) {
     // every load of the round goes out before the first product (left to itself the
     // compiler sinks each load to its use: 7.3 instead of 5.4 us for 48 x 512 x 512)
     __builtin_amdgcn_sched_barrier(0);
+    // Sums of 4 products (one value of the chunk's 16-byte pieces), which meet in pairs over
+    // the round, whose sum joins the running one: no more roundings on the way of a product
+    // than in the GEMV, whose lanes keep sums of K / 256 products that meet in a tree.
+    // (Four running sums over a wave's whole share of K left 1.4 times the GEMV's error at
+    // K = 512, 1.9 times at 1376 and 2.7 times at 4096; 48 x 1376 x 512 took 5.9 us with them
+    // and takes 6.1, 48 x 512 x 1376 7.8 and 8.3, 512 x 4096 x 4096 305 and 244.)
+    f32x4_t t[U][4][MT][NT];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -100,11 +104,25 @@ __global__ __launch_bounds__(kWavesF * 64) void gemm_f32_kernel(GemmF32Args p) {
         for (int i = 0; i < MT; ++i)
 #pragma unroll
           for (int j = 0; j < NT; ++j)
-            acc[e][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[u][i][e], wb[u][j][e], acc[e][i][j], 0, 0, 0);
+            t[u][e][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[u][i][e], wb[u][j][e], zero, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        f32x4_t v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = (t[u][0][i][j] + t[u][1][i][j]) + (t[u][2][i][j] + t[u][3][i][j]);
+#pragma unroll
+        for (int n = U; n > 1; n /= 2)
+#pragma unroll
+          for (int u = 0; u < n / 2; ++u) v[u] = v[2 * u] + v[2 * u + 1];
+        acc[i][j] += v[0];
+      }
   }
 
   // lane holds D[4 (lane / 16) + e][lane % 16] of each 16 x 16 tile
   constexpr int TS = 16 * NT + 1;
+  static_assert(kWavesF == 4, "summed in pairs below");
   __shared__ float part[kWavesF][16 * MT][TS];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -112,8 +130,7 @@ __global__ __launch_bounds__(kWavesF * 64) void gemm_f32_kernel(GemmF32Args p) {
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        part[wave][16 * i + kq + e][16 * j + r] =
-            (acc[0][i][j][e] + acc[1][i][j][e]) + (acc[2][i][j][e] + acc[3][i][j][e]);
+        part[wave][16 * i + kq + e][16 * j + r] = acc[i][j][e];
   __syncthreads();
   constexpr int kOut = 16 * MT * 16 * NT;
 #pragma unroll
@@ -121,9 +138,7 @@ __global__ __launch_bounds__(kWavesF * 64) void gemm_f32_kernel(GemmF32Args p) {
     const int t = tid + kWavesF * 64 * o, row = t / (16 * NT), col = t % (16 * NT);
     const int32_t gm = m0 + row, gn = n0 + col;
     if (gm >= p.M || gn >= p.N) continue;
-    float v = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kWavesF; ++w) v += part[w][row][col];
+    float v = (part[0][row][col] + part[1][row][col]) + (part[2][row][col] + part[3][row][col]);
     const int64_t idx = static_cast<int64_t>(gm) * p.N + gn;
     if (p.residual != nullptr) v = p.residual[idx] + v;
     p.out[idx] = v;

@@ -68,6 +68,25 @@ def test_linear_f32_rows(m, n, k):
     del keep
 
 
+@pytest.mark.parametrize("m,n,k", [(48, 1376, 512), (48, 512, 1376), (300, 2048, 520), (17, 4096, 8192)])
+def test_linear_f32_rows_error(m, n, k):
+    """The fp32 GEMM's error against fp64 (both tile sizes) is no larger than that of the
+    GEMV per row: rms over all elements, with 5% for the sampling of two rms of at least
+    65,000 elements each (below 1%) and the elements that share an operand row."""
+    rng = np.random.default_rng(k)
+    x, w = (dev(rng.standard_normal(s, dtype=np.float32)) for s in ((m, k), (n, k)))
+    dw, keep = pack_weight(host(w), N.AM_WF_F32)
+    ref = x.double() @ w.double().T
+    rms = []
+    for mode in (0, 1):
+        out = empty((m, n), torch.float32)
+        L.call("am_gfx950_linear", N.LinearArgs(p(x), 0, m, dw, p(out), 0, None, mode), stream())
+        assert launched().startswith("gemm_f32<" if mode == 0 else "gemv<"), launched()
+        rms.append(float((out.double() - ref).square().mean().sqrt()))
+    assert rms[0] <= 1.05 * rms[1], rms
+    del keep
+
+
 # (m, n, k, group): rows and columns on both sides of the 64-, 128- and 256-row tiles of
 # every weight format, one k step, an odd number of groups, groups of one, two and four
 # 64-value steps
