@@ -48,7 +48,8 @@ struct AttnArgs {
   int64_t cbs;  // cache batch stride (elements)
   int32_t splits;
   int32_t min_per_split;  // fewest positions one split block handles
-  int32_t short_splits;   // decode kernel: most splits of a context below kDecLong
+  int32_t rows, round, slots, even_splits;  // 8-wave decode blocks (decode_slot)
+  uint32_t even_inv;  // ceil(2^32 / d), d the divisor of even_slot
   float scale;  // log2(e) / sqrt(d)
   float* part;
   unsigned* tickets;  // [rows][hkv], zero between calls
@@ -486,7 +487,7 @@ __global__ __launch_bounds__(kWaves * 64) void attention_kernel(AttnArgs p) {
 
 // ---- decode: one query position per row, bf16 q and cache, both products on MFMA ----
 //
-// grid = (splits, kv_heads, batch).  A block of NW waves owns one (row, kv head) and a
+// grid = (splits, kv_heads, batch), or planned (decode_slot).  A block of NW waves owns one (row, kv head) and a
 // slice of positions; wave w takes the 32-position steps w, w + NW, ... of the slice,
 // with the next step's K and V loads in flight while a step computes.  NW = 4 (one
 // wave per SIMD, 264 registers) unless the grid already gives every CU a block
@@ -522,6 +523,149 @@ constexpr int64_t kDecLong = 4096;
 constexpr int32_t kDecMinPerSplit = 64;
 constexpr int kDecMaxSplits = 8;
 
+__device__ __forceinline__ float lane_value(float v, int from) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), from));
+}
+// Sum and maximum over a wave.
+__device__ __forceinline__ float wave_sum(float v, int lane) {
+  v = group_sum<16>(v);
+  v += xor_partner<16>(v, lane);
+  return lane_value(v + xor_partner<32>(v, lane), 0);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v) {
+  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false)));
+}
+__device__ __forceinline__ float wave_max(float v, int lane) {
+  v = dpp_max<0x140>(dpp_max<0x141>(dpp_max<0x4E>(dpp_max<0xB1>(v))));
+  v = fmaxf(v, xor_partner<16>(v, lane));
+  return lane_value(fmaxf(v, xor_partner<32>(v, lane)), 0);
+}
+// Sum over the lanes up to and including this one (row_shr 1, 2, 4, 8, row_bcast 15, 31).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_shift_add(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROWS, 0xF, false));
+}
+__device__ __forceinline__ float wave_scan(float v) {
+  v = dpp_shift_add<0x118, 0xF>(dpp_shift_add<0x114, 0xF>(dpp_shift_add<0x112, 0xF>(dpp_shift_add<0x111, 0xF>(v))));
+  return dpp_shift_add<0x143, 0xC>(dpp_shift_add<0x142, 0xA>(v));
+}
+
+// Which (row, split) the 8-wave decode block `slot` of a kv head takes.  One such block fits
+// a CU, so a launch has `round` of them at once per kv head, and a block costs about as much
+// again as kDecBlockKeys positions (16 rows at contexts 400-777: 8 splits in four rounds 24.0
+// us, 2 in one 12.0).  Every block derives the same plan from the contexts of all rows:
+//   * near-equal contexts: even_splits (as many as one round holds) for every row;
+//   * otherwise (an even split leaves the longest slice a third above what the round could
+//     have): the shortest slice with which all rows fit the round, so long rows take more
+//     splits than short ones; and where a round has no blocks to spare for them, up to
+//     kDecSpare blocks beyond it (or a second round of long contexts: 12 rows at 4000-8000
+//     66 us in one, 64 in two) if that ends earlier by the same count of positions.  Split
+//     rows come first.
+// Calls whose rows all may have their most splits in one round have nothing to plan.
+// One row at 16384 positions among 15 at 300 (cold caches, launch included): 113 us with the
+// even split, 50 so, 47 with 8 splits for every row; among 31 201, 56 and 69; 16 rows spread
+// over 50-4000 43, 35 and 41.  Where the split stays even the plan costs 0.2-0.5 us (16 rows
+// at 400-777 23.2 -> 23.6).
+constexpr float kDecBlockKeys = 400.0f;
+constexpr int kDecSpare = 8;
+constexpr float kDecUneven = 1.33f;
+struct DecodeSlot {
+  int row, split, splits;  // of the row; row < 0: no work
+  int32_t keys;
+};
+// The even split's (row, split) of a slot: splits of a row side by side, or where there are
+// more slots than a round all rows' first splits first.  (row >= rows, split >= even_splits:
+// no work)
+__device__ __forceinline__ void even_slot(const AttnArgs& p, uint32_t slot, int& row, int& split) {
+  const uint32_t d = p.slots <= p.round ? p.even_splits : p.rows;
+  const uint32_t q = d == 1 ? slot : __umulhi(slot, p.even_inv), r = slot - q * d;  // (slot / d)
+  row = static_cast<int>(p.slots <= p.round ? q : r);
+  split = static_cast<int>(p.slots <= p.round ? r : q);
+}
+__device__ __forceinline__ DecodeSlot decode_slot(const AttnArgs& p, int slot, int lane) {
+  const int B = p.rows;
+  // (the capacity is below 2^31)
+  auto row_len = [&](int r) { return static_cast<int32_t>(row_keys(p, r, 0)); };
+  auto keys = [&](int r) { return fmaxf(static_cast<float>(row_len(r)), 1.0f); };
+  const int32_t len0 = lane < B ? row_len(lane) : 0;  // rows past the first 64 are read where needed
+  const float k0 = lane < B ? fmaxf(static_cast<float>(len0), 1.0f) : 0.0f;
+  auto take = [&](int row, int split, int splits) -> DecodeSlot {
+    return {row, split, splits, row < 64 ? __builtin_amdgcn_readlane(len0, row) : row_len(row)};
+  };
+  float total = k0, most = k0;
+  for (int r = lane + 64; r < B; r += 64) {
+    total += keys(r);
+    most = fmaxf(most, keys(r));
+  }
+  total = wave_sum(total, lane);
+  most = wave_max(most, lane);
+  const float fb = static_cast<float>(B), fr = static_cast<float>(p.round), fs = static_cast<float>(p.splits);
+  // what the blocks of the even split take at most, and what any split could reach
+  const float even = most / static_cast<float>(p.even_splits);
+  const float ideal = B <= p.round ? total / fr : ceilf(fb / fr) * (total / fb + kDecBlockKeys) - kDecBlockKeys;
+  float len = 0.0f;  // slice length, 0: the even split
+  if (__builtin_expect(even > kDecUneven * fmaxf(ideal, most / fs) + 192.0f, 0)) {
+    auto chunk = [&](int r0) { return r0 == 0 ? k0 : r0 + lane < B ? keys(r0 + lane) : 0.0f; };
+    // blocks of slices of l >= most / splits positions: one per row, and one more for each
+    // multiple of l below its context
+    auto blocks = [&](float l) {
+      int n = B;
+      for (int r0 = 0; r0 < B; r0 += 64) {
+        const float k = chunk(r0);
+#pragma unroll
+        for (int i = 1; i < kDecMaxSplits; ++i)
+          n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(k > l * static_cast<float>(i)));
+      }
+      return n;
+    };
+    // slice with which at most `limit` blocks are needed, to a sixteenth; hi's are few enough
+    auto shortest = [&](int limit, float least, float enough) {
+      int lo = static_cast<int>(ceilf(fmaxf(least, most / fs) / 32.0f)), hi = static_cast<int>(ceilf(enough / 32.0f));
+      if (lo >= hi || blocks(32.0f * lo) <= limit) return 32.0f * lo;
+      while (hi - lo > 1 + lo / 16) {
+        const int mid = (lo + hi) / 2;
+        if (blocks(32.0f * mid) <= limit) hi = mid;
+        else lo = mid;
+      }
+      return 32.0f * hi;
+    };
+    float end = fmaxf(most, ideal) + kDecBlockKeys;
+    if (B <= p.round) {
+      len = shortest(p.round, ideal, even);
+      end = len + kDecBlockKeys;
+    }
+    if (p.slots > p.round) {
+      const float l = shortest(p.slots, total / static_cast<float>(p.slots), most), n = static_cast<float>(blocks(l));
+      if (fmaxf(l + kDecBlockKeys, ceilf(n / fr) * (total / n + kDecBlockKeys)) < end) len = l;
+    }
+    if (len > 0.0f) {
+      // rows of several splits, then rows of one
+      float at = static_cast<float>(slot);
+      for (int pass = 0; pass < 2; ++pass) {
+        for (int r0 = 0; r0 < B; r0 += 64) {
+          const float k = chunk(r0);
+          float n = k > 0.0f ? 1.0f : 0.0f;
+#pragma unroll
+          for (int i = 1; i < kDecMaxSplits; ++i) n += k > len * static_cast<float>(i) ? 1.0f : 0.0f;
+          const float mine = (n > 1.0f) == (pass == 0) ? n : 0.0f;
+          const float upto = wave_scan(mine), all = lane_value(upto, 63);
+          if (at < all) {
+            const int i = __builtin_popcountll(__builtin_amdgcn_ballot_w64(upto <= at));
+            const float n_row = lane_value(mine, i);
+            return take(r0 + i, static_cast<int>(at - (lane_value(upto, i) - n_row)), static_cast<int>(n_row));
+          }
+          at -= all;
+        }
+      }
+      return {-1, 0, 1, 0};
+    }
+  }
+  int row, split;
+  even_slot(p, slot, row, split);
+  return row < B && split < p.even_splits ? take(row, split, p.even_splits) : DecodeSlot{-1, 0, 1, 0};
+}
+
 // NW = 8: two waves per SIMD (236 VGPRs, no spills, against 264 for the 4-wave block,
 // which holds one wave per SIMD), for grids that already give every CU a block.
 template <int D, int G, int NW>
@@ -539,25 +683,34 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(AttnArgs p) {
   const int j = lane & 15, h = lane >> 4;
   typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
   typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-  // Grid (splits, kv heads, rows), or (kv heads, rows, splits) where a context may use
-  // fewer splits than the grid has: the live blocks then come first and spread over the
-  // XCDs (block i runs on XCD i mod 8; 16 rows at contexts 400-777, 2 of 4 splits live: 18.4
-  // us with the splits first, 12.6 us).
-  const bool live_first = p.short_splits < p.splits;
-  const int64_t qr = live_first ? blockIdx.y : blockIdx.z;
-  const int64_t b = qr / p.seq, s = qr % p.seq;
-  const int64_t g = live_first ? blockIdx.x : blockIdx.y;
-  const int split = live_first ? blockIdx.z : blockIdx.x;
-  const int64_t n_keys = row_keys(p, b, s);
+  // Grid (splits, kv heads, rows); 8-wave blocks: (slots, kv heads), or where they are more
+  // than one round (kv heads, slots), whose first slots are the long rows'.
+  int64_t g = blockIdx.y;
+  DecodeSlot at;
+  if (NW > kDecWaves && p.slots > 0) {
+    const bool many = p.slots > p.round;
+    at = decode_slot(p, static_cast<int>(many ? blockIdx.y : blockIdx.x), lane);
+    if (at.row < 0) return;
+    if (many) g = blockIdx.x;
+    at.row = __builtin_amdgcn_readfirstlane(at.row);  // (the compiler takes them for lane values)
+    at.split = __builtin_amdgcn_readfirstlane(at.split);
+    at.splits = __builtin_amdgcn_readfirstlane(at.splits);
+    at.keys = __builtin_amdgcn_readfirstlane(at.keys);
+  } else {
+    at = {static_cast<int>(blockIdx.z), static_cast<int>(blockIdx.x), p.splits, static_cast<int32_t>(row_keys(p, blockIdx.z, 0))};
+  }
+  const int64_t qr = at.row, b = qr;
+  const int split = at.split;
+  const uint32_t n_keys = static_cast<uint32_t>(max(at.keys, 0));
   // Slices are whole 32-position steps (a step then never straddles two cache blocks):
   // the slice length is rounded up to 32 and the live split count follows from it,
   // the same in every block of the (row, kv head).
-  const int64_t ns0 = live_splits(n_keys, n_keys < kDecLong ? p.short_splits : p.splits, p.min_per_split);
-  const int64_t per = (((n_keys + ns0 - 1) / ns0) + 31) & ~int64_t{31};
-  const int64_t nsplit = (n_keys + per - 1) / per;
+  const uint32_t ns0 = max(min((n_keys + p.min_per_split - 1) / p.min_per_split, static_cast<uint32_t>(at.splits)), 1u);
+  const uint32_t per = max(((n_keys + ns0 - 1) / ns0 + 31) & ~31u, 32u);
+  const int64_t nsplit = max((n_keys + per - 1) / per, 1u);
   if (split >= nsplit) return;  // surplus block for this context
-  const int64_t lo = split * per;
-  const int64_t hi = lo + per < n_keys ? lo + per : n_keys;
+  const int64_t lo = static_cast<int64_t>(split) * per;
+  const int64_t hi = min(lo + per, static_cast<int64_t>(n_keys));
   const int64_t nsteps = (hi - lo + 31) / 32;
   const int64_t my = nsteps > wave ? (nsteps - wave + NW - 1) / NW : 0;  // this wave's steps
 
@@ -1453,25 +1606,29 @@ extern "C" am_status_code am_gfx950_attention(const am_gfx950_attention_args* a,
     p.min_per_split = a->num_splits > 0 ? 32 : kDecMinPerSplit;
     if (a->num_splits <= 0 && p.splits > kDecMaxSplits) p.splits = kDecMaxSplits;
     // Grids that give every CU a block run 8-wave blocks, two waves per SIMD: twice the
-    // K/V loads in flight per CU, merged in LDS.  One such block fits a CU and more run in
-    // rounds, so the splits are cut to one round of blocks: 16 rows at contexts 400-777
-    // 24.0 -> 12.0 us, 1000-2000 32.4 -> 23.3, 4000-8000 84.0 -> 81.6; 5 rows at 4000-8000
-    // 35.5 -> 30.6.  Where one round leaves more than an eighth of the CUs idle and two
-    // rounds do not, contexts of kDecLong positions take two (12 rows at 4000-8000: 65.1
-    // us with 8 splits, 67.0 in one round, 64.3 in two).
+    // K/V loads in flight per CU, merged in LDS.  Their splits follow the contexts
+    // (decode_slot).
     const int64_t pairs = a->hkv * batch, cus = DeviceCUs();
-    const bool wide = a->num_splits <= 0 && pairs * p.splits >= cus;
-    p.short_splits = p.splits;
-    if (wide) {
-      const int64_t one = std::max<int64_t>(1, std::min<int64_t>(p.splits, cus / pairs));
-      const int64_t two = std::max<int64_t>(1, std::min<int64_t>(p.splits, 2 * cus / pairs));
-      p.short_splits = static_cast<int32_t>(one);
-      p.splits = static_cast<int32_t>(8 * one * pairs < 7 * cus && 8 * two * pairs >= 14 * cus ? two : one);
-    }
-    const unsigned ns = static_cast<unsigned>(p.splits), nh = static_cast<unsigned>(a->hkv), nb = static_cast<unsigned>(batch);
-    const dim3 grid = p.short_splits < p.splits ? dim3(nh, nb, ns) : dim3(ns, nh, nb);
-    if (wide)
+    if (a->num_splits <= 0 && pairs * p.splits >= cus) {
+      const int64_t round = std::max<int64_t>(1, cus / a->hkv);
+      const int64_t even = std::max<int64_t>(1, std::min<int64_t>(p.splits, round / batch));
+      const int64_t twice = std::max<int64_t>(1, std::min<int64_t>(p.splits, 2 * round / batch));
+      int64_t slots = round;
+      if (even == p.splits) slots = 0;  // as many as a row may have: nothing to plan
+      else if (batch + kDecSpare > round) slots = std::min(batch + kDecSpare, kMaxRows);
+      else if (a->capacity >= kDecLong && 8 * even * pairs < 7 * cus && 8 * twice * pairs >= 14 * cus) slots = 2 * round;
+      p.rows = static_cast<int32_t>(batch);
+      p.round = static_cast<int32_t>(round);
+      p.slots = static_cast<int32_t>(slots);
+      p.even_splits = static_cast<int32_t>(even);
+      p.even_inv = static_cast<uint32_t>(CeilDiv(int64_t{1} << 32, slots <= round ? even : batch));
+      const unsigned ns = static_cast<unsigned>(slots), nh = static_cast<unsigned>(a->hkv);
+      const dim3 grid = slots == 0     ? dim3(static_cast<unsigned>(p.splits), nh, static_cast<unsigned>(batch))
+                        : slots > round ? dim3(nh, ns)
+                                        : dim3(ns, nh);
       return a->head_dim == 128 ? LaunchDecode<128, 8>(G, grid, p, s) : LaunchDecode<64, 8>(G, grid, p, s);
+    }
+    const dim3 grid(static_cast<unsigned>(p.splits), static_cast<unsigned>(a->hkv), static_cast<unsigned>(batch));
     return a->head_dim == 128 ? LaunchDecode<128, kDecWaves>(G, grid, p, s)
                               : LaunchDecode<64, kDecWaves>(G, grid, p, s);
   }

@@ -201,6 +201,40 @@ def test_attention_decode_split_rounds(B, hkv, paged):
             assert bool((err <= ref.abs() * 2.0 ** -8 + 2.0 ** -15 * vr.abs().max()).all()), (r, n)
 
 
+@pytest.mark.parametrize("B,hkv", [(16, 8), (24, 8), (32, 8), (100, 8), (9, 24)])
+@pytest.mark.parametrize("at", [0, -1])
+def test_attention_decode_one_long_row(B, hkv, at):
+    """One long context among short ones keeps its 8 splits whatever the batch (the records
+    written to the workspace tell them; the short rows are one block each), against fp64
+    attention.  Twice on one workspace, whose tickets are left zero."""
+    g, d, cap, long = 4, 128, 4608, 4600
+    hq, gen = g * hkv, torch.Generator("cuda").manual_seed(B)
+    lens = [1 + (7 * r) % 60 for r in range(B)]
+    lens[at] = long
+    k, v = (torch.randn((B, hkv, cap, d), device="cuda", generator=gen).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn((B, hq * d), device="cuda", generator=gen).to(torch.bfloat16)
+    posd = dev(np.array(lens, np.int64) - 1)
+    wsb = L.am_gfx950_attention_workspace_bytes(B, 1, hq, hkv, d, cap, 0)
+    tickets = 64 * -(-B * hkv * 4 // 256)
+    for _ in range(2):
+        ws = torch.full((wsb // 4,), 0x7FC0DEAD, dtype=torch.int32, device="cuda")
+        ws[:tickets] = 0
+        out = empty((B, hq * d), torch.bfloat16)
+        L.call("am_gfx950_attention", N.AttentionArgs(p(q), p(k), p(v), p(out), 1, hq, hkv, d, cap, 0, p(posd), B,
+                                                      hkv * cap * d, 1, 0, p(ws), wsb), stream())
+        assert not bool(ws[:tickets].any())
+        # a record: maximum, sum and d outputs of g heads
+        assert int((ws[tickets:] != 0x7FC0DEAD).sum()) == 8 * hkv * g * (d + 2)
+        for r in sorted({0, 1, B // 2, B - 1}):
+            n = lens[r]
+            kr, vr = (t[r, :, :n].double().repeat_interleave(g, 0) for t in (k, v))
+            sc = (kr * q[r].double().view(hq, 1, d)).sum(-1) / d ** 0.5
+            ref = (torch.softmax(sc, -1).unsqueeze(-1) * vr).sum(1).view(-1)
+            err = (out[r].double() - ref).abs()
+            # a bf16 rounding of the output and P in bf16 hi + lo (2^-16 of the row's largest value)
+            assert bool((err <= ref.abs() * 2.0 ** -8 + 2.0 ** -15 * vr.abs().max()).all()), (r, n)
+
+
 @pytest.mark.parametrize("m,n,k", [(6, 4096, 14336), (16, 40, 14336), (9, 17, 16384), (16, 128, 5632)])
 @pytest.mark.parametrize("fmt", [N.AM_WF_INT4, N.AM_WF_INT8, N.AM_WF_BF16])
 def test_batched_rows_past_lds(m, n, k, fmt):
