@@ -521,6 +521,26 @@ void TestKVBlocks() {
   CHECK(m.EnsureCapacity(1, 64 * 3).code() == StatusCode::kResourceExhausted);
 }
 
+// A workspace sized for the longest chunk serves every shorter one: the bytes never fall as
+// the rows grow, although long launches split less than short ones or not at all.
+void TestGemmWorkspace() {
+  const int64_t shapes[][3] = {{6144, 4096, 128}, {4096, 4096, 128}, {28672, 4096, 128}, {4096, 14336, 128},
+                               {520, 4096, 64},   {130, 2048, 128},  {1000, 8192, 256},  {4096, 512, 128}};
+  for (const auto& s : shapes) {
+    int64_t before = 0;
+    bool grows = true;
+    for (int64_t m = 1; m <= 5000; m += m < 600 ? 1 : 37) {
+      const int64_t bytes = am_gfx950_gemm_workspace_bytes(m, s[0], s[1], s[2]);
+      grows = grows && bytes >= before;
+      before = bytes;
+    }
+    CHECK(grows);
+  }
+  CHECK(am_gfx950_gemm_workspace_bytes(4096, 4096, 14336, 128) >= am_gfx950_gemm_workspace_bytes(37, 4096, 14336, 128));
+  CHECK(am_gfx950_gemm_workspace_bytes(37, 4096, 14336, 128) > 0);
+  CHECK(am_gfx950_gemm_workspace_bytes(4096, 4096, 512, 128) == 0);
+}
+
 int main() {
   TestKVBlocks();
   TestPackedCacheHeader();
@@ -528,6 +548,7 @@ int main() {
   TestKV();
   TestExecutor();
   TestGfx950Registrations();
+  TestGemmWorkspace();
   std::printf("%d checks, %d failures\n", g_checks, g_failures);
   return g_failures == 0 ? 0 : 1;
 }

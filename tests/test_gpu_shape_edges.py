@@ -162,6 +162,26 @@ def test_prefill_gemm_zero_scale_groups(m, n, k, group, size):
     assert not bool(out[:, 5::40].any())
 
 
+@pytest.mark.parametrize("fmt", [N.AM_WF_INT4, N.AM_WF_INT8, N.AM_WF_BF16])
+def test_prefill_gemm_workspace_of_longer_chunk(fmt):
+    """A short prompt splits K in the workspace of a session whose chunks are long enough
+    never to split, to the bits of its own workspace's result."""
+    m, n, k = 37, 1024, 14336
+    rng = np.random.default_rng(37)
+    dw, keep = pack_weight(rbf(rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02)), fmt)
+    xd = bf16_dev(bf16_rne_bits(act_rows(9, m, k)))
+    outs = []
+    for rows in (m, 12288):
+        nbytes = L.am_gfx950_gemm_workspace_bytes(rows, n, k, 128)
+        ws = torch.zeros(max(nbytes, 16), dtype=torch.uint8, device="cuda")
+        outs.append(empty((m, n), torch.bfloat16))
+        args = N.LinearArgs(p(xd), N.AM_DT_BF16, m, dw, p(outs[-1]), N.AM_DT_BF16, None, 2, p(ws), nbytes)
+        L.call("am_gfx950_linear", args, stream())
+        assert "splits=8" in launched(), launched()
+    assert torch.equal(outs[0], outs[1])
+    del keep
+
+
 @pytest.mark.parametrize("B,hkv", [(16, 8), (12, 8), (9, 8), (5, 8), (64, 8), (24, 2)])
 @pytest.mark.parametrize("paged", [False, True])
 def test_attention_decode_split_rounds(B, hkv, paged):
