@@ -1388,9 +1388,10 @@ void LaunchPrefillG(AttnArgs a, int64_t batch, int64_t ws_bytes, hipStream_t s) 
   auto blocks = [&](int64_t qb) { return CeilDiv(a.seq, qb) * per; };
   constexpr int QT = 16 / G;
   // (a 512-thread block needs a whole 16-byte piece per thread per tile: D = 128)
-  if (D == 128 && blocks(16 * QT) >= cus)
-    LaunchPrefillShape<D, G, 2, D == 128 ? 8 : 4, 1>(blocks(16 * QT), a, s);
-  else if (blocks(8 * QT) >= cus)
+  if constexpr (D == 128) {
+    if (blocks(16 * QT) >= cus) return LaunchPrefillShape<D, G, 2, 8, 1>(blocks(16 * QT), a, s);
+  }
+  if (blocks(8 * QT) >= cus)
     LaunchPrefillShape<D, G, 2, 4, 2>(blocks(8 * QT), a, s);
   else {
     const int64_t nb = blocks(4 * QT);

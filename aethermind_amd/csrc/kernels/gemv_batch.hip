@@ -535,10 +535,9 @@ int64_t BatchRowsFit(const am_gfx950_weight& w, int tpb) {
   return 0;
 }
 
-// Shape / format checks shared by every batched entry; fills the weight fields and
-// returns the dynamic LDS bytes through *lds.
+// Shape / format checks shared by every batched entry; fills the weight fields.
 am_status_code PrepareBatch(const am_gfx950_weight& w, int64_t rows, const void* x, int64_t x_stride, int tpb,
-                            BatchArgs* a, size_t* lds) {
+                            BatchArgs* a) {
   AM_CHECK_ARG(rows >= 1 && rows <= kBatchMaxRows, "batched decode: rows must be 1..16");
   AM_CHECK_ARG(w.data != nullptr && w.n > 0 && w.k > 0 && w.n < (int64_t{1} << 30) && w.k < (int64_t{1} << 30),
                "batched decode: bad weight shape");
@@ -562,21 +561,26 @@ am_status_code PrepareBatch(const am_gfx950_weight& w, int64_t rows, const void*
   a->k = static_cast<int32_t>(w.k);
   a->rows = static_cast<int32_t>(rows);
   a->row_bytes = w.format == AM_WF_BF16 ? 2 * w.k : (w.format == AM_WF_INT8 ? w.k : w.k / 2);
-  *lds = BatchLdsOf(w, std::min<int64_t>(rows, BatchRowsFit(w, tpb)), tpb);
   return AM_STATUS_OK;
 }
 
-// Runs launch(args, lds) over groups of token rows small enough for one block's LDS
-// (every group re-reads the weights; 16 rows of the 8B shapes' 4096 values fit).  off(args,
-// g0) moves the group's row pointers (outputs, positions) to row g0.  Rows that are only
-// multiplied (one tile per unit, no norm) run as one launch whatever their length: past
-// the LDS the kernel reads them from memory (XG).  The 8B down projection (k = 14336, 5
-// rows fit), INT4 / INT8 / bf16: 8 rows 28.3 / 35.7 / 62.2 -> 19.8 / 20.2 / 33.6 us, 16 rows
-// 56.3 / 70.1 / 122.7 -> 26.5 / 25.6 / 42 us.  Rows that fit stay in LDS (4 rows INT4
-// 14.4 us against 16.9).
+// Rows that are only multiplied (one tile per unit, no norm) run as one launch whatever
+// their length: past the LDS the kernel reads them from memory (XG).  The 8B down projection
+// (k = 14336, 5 rows fit), INT4 / INT8 / bf16, against groups of rows that fit, each of which
+// reads the weights again: 8 rows 28.3 / 35.7 / 62.2 -> 19.8 / 20.2 / 33.6 us, 16 rows 56.3 /
+// 70.1 / 122.7 -> 26.5 / 25.6 / 42 us.  Rows that fit stay in LDS (4 rows INT4 14.4 us against
+// 16.9).
+template <int EPI>
+am_status_code LaunchRows(const BatchArgs& a, const am_gfx950_weight& w, hipStream_t s) {
+  return DispatchBatch<EPI, false, 1>(w.format, a, BatchLdsOf(w, a.rows, 1), s);
+}
+
+// Runs launch(args, lds) over groups of normalised token rows small enough for one block's
+// LDS (every group re-reads the weights; 16 rows of the 8B shapes' 4096 values fit).
+// off(args, g0) moves the group's row pointers (outputs, positions) to row g0.
 template <class Launch, class Offset>
 am_status_code ForRowGroups(const BatchArgs& a, const am_gfx950_weight& w, int tpb, Launch launch, Offset off) {
-  const int64_t per = tpb == 1 && a.norm_w == nullptr ? a.rows : std::min<int64_t>(a.rows, BatchRowsFit(w, tpb));
+  const int64_t per = std::min<int64_t>(a.rows, BatchRowsFit(w, tpb));
   for (int64_t g0 = 0; g0 < a.rows; g0 += per) {
     BatchArgs ga = a;
     ga.rows = static_cast<int32_t>(std::min<int64_t>(per, a.rows - g0));
@@ -608,32 +612,24 @@ bool BatchLinearEligible(int32_t act, const am_gfx950_weight& w, int64_t m, cons
 am_status_code BatchLinear(const void* x, int64_t m, const am_gfx950_weight& w, void* out, int32_t out_dtype,
                            const void* residual, hipStream_t s) {
   BatchArgs a{};
-  size_t lds = 0;
-  if (auto st = PrepareBatch(w, m, x, w.k, 1, &a, &lds); st != AM_STATUS_OK) return st;
+  if (auto st = PrepareBatch(w, m, x, w.k, 1, &a); st != AM_STATUS_OK) return st;
   AM_CHECK_ARG(out != nullptr, "linear: null output");
   a.out = out;
   a.out_stride = w.n;
   a.out_f32 = out_dtype == AM_DT_F32 ? 1 : 0;
   a.units = static_cast<int32_t>(CeilDiv(w.n, 16));
-  auto off = [&](BatchArgs& g, int64_t g0) {
-    g.out = static_cast<uint8_t*>(out) + g0 * a.out_stride * (a.out_f32 ? 4 : 2);
-    if (g.residual != nullptr) g.residual = a.residual + g0 * a.res_stride;
-  };
   if (residual != nullptr) {
     AM_CHECK_ARG(out_dtype == AM_DT_BF16, "linear: residual needs out dtype == activation dtype");
     a.residual = static_cast<const uint16_t*>(residual);
     a.res_stride = w.n;
-    return ForRowGroups(a, w, 1, [&](const BatchArgs& g, size_t l) {
-      return DispatchBatch<kBResidual, false, 1>(w.format, g, l, s); }, off);
+    return LaunchRows<kBResidual>(a, w, s);
   }
-  return ForRowGroups(a, w, 1, [&](const BatchArgs& g, size_t l) {
-    return DispatchBatch<kBStore, false, 1>(w.format, g, l, s); }, off);
+  return LaunchRows<kBStore>(a, w, s);
 }
 
 am_status_code BatchQkv(const am_gfx950_fused_qkv_args* q, hipStream_t s) {
   BatchArgs a{};
-  size_t lds = 0;
-  if (auto st = PrepareBatch(q->w_qkv, q->rows, q->h, q->w_qkv.k, 2, &a, &lds); st != AM_STATUS_OK) return st;
+  if (auto st = PrepareBatch(q->w_qkv, q->rows, q->h, q->w_qkv.k, 2, &a); st != AM_STATUS_OK) return st;
   AM_CHECK_ARG(q->dtype == AM_DT_BF16, "fused_qkv: batched rows need bf16 activations");
   AM_CHECK_ARG(q->head_dim % 32 == 0, "fused_qkv: batched rows need head_dim % 32 == 0");
   AM_CHECK_ARG(Aligned16(q->norm_w), "fused_qkv: norm weight must be 16-byte aligned");
@@ -663,26 +659,19 @@ am_status_code BatchQkv(const am_gfx950_fused_qkv_args* q, hipStream_t s) {
 
 am_status_code BatchLinearResidual(const am_gfx950_fused_linear_residual_args* r, hipStream_t s) {
   BatchArgs a{};
-  size_t lds = 0;
-  if (auto st = PrepareBatch(r->w, r->rows, r->x, r->w.k, 1, &a, &lds); st != AM_STATUS_OK) return st;
+  if (auto st = PrepareBatch(r->w, r->rows, r->x, r->w.k, 1, &a); st != AM_STATUS_OK) return st;
   AM_CHECK_ARG(r->dtype == AM_DT_BF16, "fused_linear_residual: batched rows need bf16 activations");
   a.out = r->h;
   a.out_stride = r->w.n;
   a.residual = static_cast<const uint16_t*>(r->h);
   a.res_stride = r->w.n;
   a.units = static_cast<int32_t>(CeilDiv(r->w.n, 16));
-  return ForRowGroups(a, r->w, 1, [&](const BatchArgs& g, size_t l) {
-    return DispatchBatch<kBResidual, false, 1>(r->w.format, g, l, s); },
-    [&](BatchArgs& g, int64_t g0) {
-      g.out = static_cast<uint16_t*>(a.out) + g0 * a.out_stride;
-      g.residual = a.residual + g0 * a.res_stride;
-    });
+  return LaunchRows<kBResidual>(a, r->w, s);
 }
 
 am_status_code BatchGateUp(const am_gfx950_fused_gate_up_args* gu, hipStream_t s) {
   BatchArgs a{};
-  size_t lds = 0;
-  if (auto st = PrepareBatch(gu->w_gate_up, gu->rows, gu->h, gu->w_gate_up.k, 2, &a, &lds); st != AM_STATUS_OK)
+  if (auto st = PrepareBatch(gu->w_gate_up, gu->rows, gu->h, gu->w_gate_up.k, 2, &a); st != AM_STATUS_OK)
     return st;
   AM_CHECK_ARG(gu->dtype == AM_DT_BF16, "fused_gate_up: batched rows need bf16 activations");
   AM_CHECK_ARG(gu->w_gate_up.n % 32 == 0, "fused_gate_up: batched rows need ffn % 16 == 0");
@@ -700,8 +689,7 @@ am_status_code BatchGateUp(const am_gfx950_fused_gate_up_args* gu, hipStream_t s
 // RMSNorm -> lm_head logits (fp32) for rows token rows.
 am_status_code BatchNormLogits(const am_gfx950_fused_lm_head_args* lm, hipStream_t s) {
   BatchArgs a{};
-  size_t lds = 0;
-  if (auto st = PrepareBatch(lm->w, lm->rows, lm->h, lm->w.k, 1, &a, &lds); st != AM_STATUS_OK) return st;
+  if (auto st = PrepareBatch(lm->w, lm->rows, lm->h, lm->w.k, 1, &a); st != AM_STATUS_OK) return st;
   AM_CHECK_ARG(lm->dtype == AM_DT_BF16, "fused_lm_head: batched rows need bf16 activations");
   AM_CHECK_ARG(lm->logits != nullptr, "fused_lm_head: batched rows need a logits buffer");
   AM_CHECK_ARG(Aligned16(lm->norm_w), "fused_lm_head: norm weight must be 16-byte aligned");
