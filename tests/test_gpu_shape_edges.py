@@ -15,7 +15,7 @@ if not torch.cuda.is_available():  # pragma: no cover
 
 import aethermind_amd.native as N  # noqa: E402
 import oracle_lib as O  # noqa: E402
-from gpu_util import bf16_dev, dev, empty, host, p, pack_weight, stream  # noqa: E402
+from gpu_util import bf16_dev, dev, empty, host, p, pack_weight, stream, zeros  # noqa: E402
 from test_gpu_decode_shapes import act_rows, bf16_rne_bits, launched, rbf  # noqa: E402
 
 L = N.lib()
@@ -49,8 +49,16 @@ def test_argmax_vector_edges(n, dt):
 def test_linear_f32_rows(m, n, k):
     """fp32 rows x fp32 weights: both tile sizes, ragged rows, columns and k tails.  Bar:
     fp32 sums of k products in any order differ by at most k * 2^-24 of the sum of their
-    magnitudes."""
+    magnitudes.  Small integers, whose sums are exact in any order: every bit."""
     rng = np.random.default_rng(m * n + k)
+    xi, wi, ri = (rng.integers(-8, 9, s).astype(np.float32) for s in ((m, k), (n, k), (m, n)))
+    di, keep = pack_weight(wi, N.AM_WF_F32)
+    xd, rd, out = dev(xi), dev(ri), empty((m, n), torch.float32)
+    ref = xi.astype(np.float64) @ wi.astype(np.float64).T
+    L.call("am_gfx950_linear", N.LinearArgs(p(xd), 0, m, di, p(out), 0, None, 0), stream())
+    L.call("am_gfx950_linear", N.LinearArgs(p(xd), 0, m, di, p(rd), 0, p(rd), 0), stream())
+    assert np.array_equal(host(out), ref) and np.array_equal(host(rd), ref + ri)
+    del keep
     x = rng.standard_normal((m, k), dtype=np.float32)
     w = rng.standard_normal((n, k), dtype=np.float32)
     res = rng.standard_normal((m, n), dtype=np.float32)
@@ -85,6 +93,31 @@ def test_linear_f32_rows_error(m, n, k):
         rms.append(float((out.double() - ref).square().mean().sqrt()))
     assert rms[0] <= 1.05 * rms[1], rms
     del keep
+
+
+def exact_weight(rng, n, k, fmt, group=128):
+    """A device weight of small integers with power-of-two scales (INT4: a zero one here and
+    there), and its values: products with small integers sum exactly in fp32, in any order
+    and from any partial sum that the kernels keep."""
+    if fmt == N.AM_WF_INT4:
+        codes = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+        sc = np.exp2(-rng.integers(4, 7, (n, k // group)).astype(np.float32)).astype(np.float16)
+        sc[rng.random(sc.shape) < 0.03] = 0
+        logical, scales = dev(codes), dev(sc.view(np.int16))
+        data, dsc = zeros((n * k // 2,), torch.uint8), zeros((n * (k // group),), torch.int16)
+        dw = N.Weight(p(data), p(dsc), n, k, fmt, group)
+        L.call("am_gfx950_pack_int4", N.PackInt4Args(p(logical), p(scales), dw), stream())
+        q = np.stack([codes & 15, codes >> 4], -1).reshape(n, k).astype(np.int8)
+        w = dev(np.where(q > 7, q - 16, q).astype(np.int8)).double() * dev(np.repeat(sc.astype(np.float32), group, 1)).double()
+        return dw, w, (logical, scales, data, dsc)
+    if fmt == N.AM_WF_INT8:
+        q = rng.integers(-127, 128, (n, k), dtype=np.int16)
+        sc = np.exp2(-rng.integers(4, 7, n).astype(np.float32))
+        data, dsc = dev((q + 128).astype(np.uint8)), dev(sc)
+        return N.Weight(p(data), p(dsc), n, k, fmt, 0), dev(q).double() * dsc.double()[:, None], (data, dsc)
+    w = rng.integers(-8, 9, (n, k)).astype(np.float32)
+    dw, keep = pack_weight(w, fmt)
+    return dw, dev(w).double(), keep
 
 
 # (m, n, k, group): rows and columns on both sides of the 64-, 128- and 256-row tiles of
@@ -259,29 +292,25 @@ def test_attention_decode_one_long_row(B, hkv, at):
 @pytest.mark.parametrize("fmt", [N.AM_WF_INT4, N.AM_WF_INT8, N.AM_WF_BF16])
 def test_batched_rows_past_lds(m, n, k, fmt):
     """Token rows that do not fit one block's LDS together run as one launch: Linear + Add
-    in place and the fp32 store, against the fp64 product of the dequantized weights."""
+    in place and the fp32 store.  The operands' sums are exact, so the results are the
+    rounded fp64 ones to the bit, and a k step lost or taken twice shows."""
     rng = np.random.default_rng(m + n)
-    w = rbf(rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02))
-    dw, keep = pack_weight(w, fmt)
-    if fmt == N.AM_WF_INT4:
-        pk, sc = O.quant_int4(w, 128)
-        w = O.dequant_int4(pk, sc, k, 128)
-    elif fmt == N.AM_WF_INT8:
-        w = O.dequant_int8(*O.quant_int8(w))
-    x, h = act_rows(9, m, k), act_rows(10, m, n)
+    dw, w, keep = exact_weight(rng, n, k, fmt)
+    x, h = (rng.integers(-4, 5, sh).astype(np.float32) for sh in ((m, k), (m, n)))
     xd, hd = bf16_dev(bf16_rne_bits(x)), bf16_dev(bf16_rne_bits(h))
-    ref = x.astype(np.float64) @ w.astype(np.float64).T
-    sums = k * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T)
-    if fmt == N.AM_WF_INT4:
-        sums = sums * 20  # codes enter offset by 136: the partial sums reach 136 / 7 of the products'
+    xt = dev(x).double()
+    ref = xt @ w.T
+    for step in range(0, k, 128):  # each step's share of every row and column is there to be missed
+        share = xt[:, step:step + 128] @ w[:, step:step + 128].T
+        present = (share != 0).any(0).double().mean(), (share != 0).any(1).all()
+        assert float(present[0]) > 0.5 and bool(present[1])
     L.call("am_gfx950_fused_linear_residual", N.FusedLinearResidualArgs(p(xd), dw, p(hd), N.AM_DT_BF16, m), stream())
     assert launched().endswith(",xg>"), launched()
-    got = hd.view(torch.bfloat16).view(m, n).double().cpu().numpy()
-    bar = (np.abs(ref) + np.abs(ref + h)) * 2.0 ** -8 + sums
-    assert (np.abs(got - (ref + h)) <= bar).all()
+    want = (dev(h) + ref.float().bfloat16().float()).bfloat16()
+    assert torch.equal(hd.view(torch.bfloat16).view(m, n), want)
     out = empty((m, n), torch.float32)
     L.call("am_gfx950_linear", N.LinearArgs(p(xd), N.AM_DT_BF16, m, dw, p(out), N.AM_DT_F32, None, 3), stream())
-    assert (np.abs(host(out) - ref) <= sums + 1e-30).all()
+    assert launched().endswith(",xg>") and torch.equal(out.double(), ref)
     del keep
 
 
