@@ -120,9 +120,9 @@ def exact_weight(rng, n, k, fmt, group=128):
     return dw, dev(w).double(), keep
 
 
-# (m, n, k, group): rows and columns on both sides of the 64-, 128- and 256-row tiles of
-# every weight format, one k step, an odd number of groups, groups of one, two and four
-# 64-value steps
+# (m, n, k, group): rows and columns on both sides of the 64- and 128-row tiles of every
+# weight format, one k step, an odd number of groups, groups of one, two and four 64-value
+# steps (the 256-row tile and the splits are pinned by test_prefill_gemm_exact)
 TILE_SHAPES = [(1, 64, 128, 128), (65, 72, 384, 128), (256, 4104, 640, 128), (257, 16392, 384, 128),
                (513, 28680, 512, 256), (300, 8200, 1024, 64), (1030, 6152, 2048, 128)]
 
@@ -160,6 +160,87 @@ def test_prefill_gemm_tiles(shape, fmt):
         err = (out.double() - ref).abs()
         bar = ref.abs() * 2.0 ** -8 + mag * (k * 2.0 ** -24) + 1e-30
         assert bool((err <= bar).all()), (launched(), float((err - bar).max()))
+    del keep
+
+
+# (epilogue, m, n, k), and the (tile rows, tile columns, splits) it reaches: all formats, or
+# INT4 and INT8, then bf16.  Ragged rows and columns in every tile; the 8B down projection
+# and chunks of its kind are where the 256-row tile and its splits are used.
+ALL = (N.AM_WF_INT4, N.AM_WF_INT8, N.AM_WF_BF16)
+EXACT_TILES = [("store", 100, 1032, 14336, (64, 64, 8)), ("residual", 65, 72, 2048, (64, 64, 2)),
+               ("silu", 100, 2048, 4096, (64, 128, 4)), ("store", 300, 2168, 8192, (128, 128, 4)),
+               ("residual", 515, 4104, 14336, (128, 256, 2), (256, 256, 4)), ("silu", 750, 28672, 512, (128, 256, 1)),
+               ("store", 1030, 12296, 512, (256, 256, 1)), ("residual", 1030, 4088, 14336, (256, 256, 2)),
+               ("silu", 1000, 28672, 512, (256, 256, 1))]
+
+
+@pytest.mark.skipif(torch.cuda.get_device_properties(0).multi_processor_count != 256, reason="tiles of 256 CUs")
+@pytest.mark.parametrize("case", EXACT_TILES, ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}-{c[3]}")
+@pytest.mark.parametrize("fmt", ALL)
+def test_prefill_gemm_exact(case, fmt):
+    """Operands whose sums are exact: a store is the rounded product to the bit, a residual
+    the rounded sum, SiLU-Mul within a rounding and fp32 exponentials of the value from the
+    rounded halves.  The launch's grid and name tell the tile; twice on one workspace."""
+    epi, m, n, k = case[:4]
+    bm, bn, splits = case[-1] if fmt == N.AM_WF_BF16 else case[4]
+    rng = np.random.default_rng(m + n)
+    dw, w, keep = exact_weight(rng, n, k, fmt)
+    x, h = (rng.integers(-4, 5, sh).astype(np.float32) for sh in ((m, k), (m, n)))
+    xd, acc = bf16_dev(bf16_rne_bits(x)), (dev(x).double() @ w.T).float().bfloat16()
+    nbytes = L.am_gfx950_gemm_workspace_bytes(m, n, k, 128)
+    ws = zeros((max(nbytes, 16),), torch.uint8)
+    none = (N.vp * 3)(None, None, None)
+    for _ in range(2):
+        if epi == "silu":
+            out = empty((m, n // 2), torch.bfloat16)
+            none[0] = p(out)
+            L.call("am_gfx950_prefill_linear", N.PrefillLinearArgs(p(xd), m, dw, N.AM_PREFILL_SILU_MUL, none, (N.i64 * 2)(0, 0),
+                                                                   p(ws), nbytes, None), stream())
+            gate, up = acc[:, :n // 2].double(), acc[:, n // 2:].double()
+            ref = torch.nn.functional.silu(gate) * up
+            # (where fp32's exponential overflows silu is below 2^-121, and 0)
+            bar = ref.abs() * (2.0 ** -8 + 2.0 ** -20) + up.abs() * 2.0 ** -121
+            over = int(((out.double() - ref).abs() > bar).sum())
+            assert over == 0, over
+        else:
+            out = bf16_dev(bf16_rne_bits(h)).view(torch.bfloat16).view(m, n)
+            res = p(out) if epi == "residual" else None
+            L.call("am_gfx950_linear", N.LinearArgs(p(xd), N.AM_DT_BF16, m, dw, p(out), N.AM_DT_BF16, res, 2, p(ws), nbytes),
+                   stream())
+            ref = (dev(h) + acc.float()).bfloat16() if res else acc
+            assert torch.equal(out, ref), int((out != ref).sum())
+        info = N.last_launch()
+        tiles = -(-m // bm) * -(-n // bn)
+        assert f"bn={bn},splits={splits}>" in info.kernel.decode() and info.grid == tiles * splits, (info.kernel, info.grid)
+        assert not bool(ws[:4096].any())
+    del keep
+
+
+@pytest.mark.parametrize("fmt", ALL)
+def test_prefill_gemm_rope_largest_tile(fmt):
+    """The q|k|v epilogue in the 256 x 256 tile with a ragged last row tile: bit for bit the
+    column split, am_gfx950_rope and am_gfx950_kv_update."""
+    m, start, cap, hq, hkv, d, H = 2049, 63, 2176, 32, 8, 128, 512
+    rng = np.random.default_rng(12)
+    dw, w, keep = exact_weight(rng, (hq + 2 * hkv) * d, H, fmt)
+    xd = bf16_dev(bf16_rne_bits(rng.integers(-4, 5, (m, H)).astype(np.float32)))
+    cd, sd = (dev(t) for t in O.rope_tables(cap, d, 10000.0))
+    startd, posd = dev(np.array([start], np.int64)), torch.arange(start, start + m, dtype=torch.int64, device="cuda")
+    planes = [zeros((hkv * cap * d,), torch.int16) for _ in range(4)]
+    qf, q, k, v = (empty((m, c * d), torch.int16) for c in (hq, hq, hkv, hkv))
+    r = N.PrefillRopeKv(p(cd), p(sd), cap, p(startd), p(planes[0]), p(planes[1]), hq, hkv, d, cap, None, None)
+    L.call("am_gfx950_prefill_linear", N.PrefillLinearArgs(p(xd), m, dw, N.AM_PREFILL_QKV_ROPE_KV, (N.vp * 3)(p(qf), None, None),
+                                                           (N.i64 * 2)(0, 0), None, 0, C.pointer(r)), stream())
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert "qkv_rope_kv,bn=256" in launched() and N.last_launch().grid == 9 * 24, launched()
+    L.call("am_gfx950_prefill_linear", N.PrefillLinearArgs(p(xd), m, dw, N.AM_PREFILL_SPLIT, (N.vp * 3)(p(q), p(k), p(v)),
+                                                           (N.i64 * 2)(hq * d, (hq + hkv) * d)), stream())
+    L.call("am_gfx950_rope", N.RopeArgs(p(q), p(k), p(q), p(k), p(posd), p(cd), p(sd), m, hq, hkv, d, cap, N.AM_DT_BF16), stream())
+    L.call("am_gfx950_kv_update", N.KvUpdateArgs(p(k), p(v), p(planes[2]), p(planes[3]), m, hkv, d, cap, 0, p(startd),
+                                                 N.AM_DT_BF16, None, None), stream())
+    assert torch.equal(qf, q) and torch.equal(planes[0], planes[2]) and torch.equal(planes[1], planes[3])
+    acc = (xd.view(torch.bfloat16).view(m, H).double() @ w.T).float().bfloat16()
+    assert torch.equal(v.view(torch.bfloat16), acc[:, (hq + hkv) * d:])
     del keep
 
 
