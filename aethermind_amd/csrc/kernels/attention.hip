@@ -487,9 +487,9 @@ __global__ __launch_bounds__(kWaves * 64) void attention_kernel(AttnArgs p) {
 
 // ---- decode: one query position per row, bf16 q and cache, both products on MFMA ----
 //
-// grid = (splits, kv_heads, batch), or planned (decode_slot).  A block of NW waves owns one (row, kv head) and a
-// slice of positions; wave w takes the 32-position steps w, w + NW, ... of the slice,
-// with the next step's K and V loads in flight while a step computes.  NW = 4 (one
+// grid = (splits, kv_heads, batch), or planned (decode_slot).  A block of NW waves owns one
+// (row, kv head) and a slice of positions; wave w takes the 32-position steps w, w + NW, ...
+// of the slice, with the next step's K and V loads in flight while a step computes.  NW = 4 (one
 // wave per SIMD, 264 registers) unless the grid already gives every CU a block
 // (batched long contexts): then NW = 8 within 236 registers, two waves per SIMD and
 // twice the K/V loads in flight per CU, the extra waves merged in LDS.

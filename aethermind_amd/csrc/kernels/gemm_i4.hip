@@ -178,7 +178,7 @@ struct I4Args {
   const uint16_t* residual;   // [M][N] bf16, may alias out0
   int32_t vec;                // 1: 16-byte output chunks (row strides and split columns % 8 == 0, aligned)
   int32_t splits;             // k splits per tile (1: none)
-  float* part;                // [tiles][splits][waves][16][64] x 4 fp32 partial accumulators
+  float* part;                // [tiles][splits][waves][MT NT][64] x 4 fp32 partial accumulators
   unsigned* tickets;          // [tiles], zero between launches
   // q|k|v + RoPE + KV epilogue: columns [0,c1) q -> out0 (rotated), [c1,c2) k (rotated)
   // and [c2,N) v into the cache planes at position *start + row
@@ -926,8 +926,10 @@ float EstimateUs(const I4Args& p, const void* ws, int64_t ws_bytes) {
   return std::max(rounds * static_cast<float>(p.K / QBK) / splits * step, weights) + merge;
 }
 
-// The tile with the smallest estimate.  The 64-row tiles take part up to 256 rows (above,
-// they read each weight more often than a launch of wider tiles of the same estimate).
+// The tile with the smallest estimate, each at the most splits that SplitsFor allows with the
+// workspace (fewer splits are not weighed against them).  The 64-row tiles take part up to
+// 256 rows (above, they read each weight more often than a launch of wider tiles of the same
+// estimate).
 template <int WF, int EPI>
 am_status_code LaunchWF(const I4Args& p, void* ws, int64_t ws_bytes, hipStream_t s) {
   constexpr int kFew = EPI == kI4SiluMul ? kT64W : kT64;

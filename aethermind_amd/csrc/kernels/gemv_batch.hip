@@ -498,7 +498,11 @@ am_status_code LaunchBatch(const BatchArgs& a, size_t lds, hipStream_t s) {
 template <int WF, int EPI, bool NORM, int TPB>
 am_status_code LaunchBatchR(const BatchArgs& a, size_t lds, hipStream_t s) {
   if constexpr (TPB == 1 && !NORM) {
-    // rows that do not fit LDS together: one launch that reads them beside the weights
+    // Rows that do not fit LDS together: one launch that reads them beside the weights.  A
+    // step of INT4 or INT8 weights loads four or two pieces of the rows with it, so 4 steps
+    // are as many loads as 8 of bf16, and the padding of a wave's share to whole rounds costs
+    // less (4 / 8 steps, cold caches, k = 14336, 16 rows: INT4 29.6 / 32.8 us, INT8 29.5 /
+    // 32.0, bf16 46.4 / 46.2; 8 rows 22.9 / 24.6, 24.3 / 26.6, 37.8 / 36.8).
     if (lds > kBatchLds) return LaunchBatch<WF, EPI, NORM, TPB, WF == AM_WF_BF16 ? 8 : 4, true>(a, lds - BatchRowBytes(a.k, a.rows), s);
   }
   if constexpr (TPB == 1) {

@@ -101,10 +101,12 @@ am_status_code am_gfx950_rmsnorm(const am_gfx950_rmsnorm_args* args, void* hip_s
 /* OpType::kLinear (linear_op.h:87-92): out[m,:] = x[m,:] @ W^T (+ residual[m,:]).
  * fp32 accumulation; out rounded once to out_dtype, and with a residual the sum is
  * rounded again (two op boundaries: Linear then Add).  residual may alias out.
- * mode: 0 auto (bf16 activations with 2 <= m <= 16 -> batched decode GEMV when the
- * weight format allows it; otherwise m <= 8 -> GEMV, else MFMA GEMM), 1 GEMV per row,
- * 2 GEMM, 3 batched decode GEMV (m <= 16, bf16 activations, bf16/int8 weights or
- * int4 with group 128; rows of k values past one block's LDS are read from memory). */
+ * mode: 0 auto (bf16 activations with 2 <= m <= 16 -> batched decode GEMV when the weight
+ * format allows it and the m rows of k values fit one block's LDS; fp32 activations and
+ * weights with m >= 2 -> fp32 MFMA GEMM, for k % 4 == 0 up to 8192 and 16-byte aligned
+ * rows; otherwise m <= 8 -> one GEMV per row, else MFMA GEMM where its k and format allow),
+ * 1 GEMV per row, 2 GEMM, 3 batched decode GEMV (m <= 16, bf16 activations, bf16/int8
+ * weights or int4 with group 128; rows past one block's LDS are read from memory). */
 typedef struct am_gfx950_linear_args {
   const void* x;
   int32_t x_dtype;
