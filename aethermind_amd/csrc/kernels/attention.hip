@@ -174,6 +174,10 @@ __device__ __forceinline__ int64_t row_keys(const AttnArgs& p, int64_t b, int64_
   const int64_t start = p.start_dev != nullptr ? p.start_dev[b] : p.start;
   return start + s + 1 <= p.cap ? start + s + 1 : p.cap;
 }
+// of a decode row, in [0, capacity] (below 2^31) whatever the position
+__device__ __forceinline__ int32_t decode_keys(const AttnArgs& p, int64_t b) {
+  return static_cast<int32_t>(max(row_keys(p, b, 0), int64_t{0}));
+}
 
 // Merge the NW per-wave states (sm_m, sm_l, sm_o) of one block, then write the output
 // (one split) or the block's partial record, and let the last split block of the
@@ -585,13 +589,11 @@ __device__ __forceinline__ void even_slot(const AttnArgs& p, uint32_t slot, int&
 }
 __device__ __forceinline__ DecodeSlot decode_slot(const AttnArgs& p, int slot, int lane) {
   const int B = p.rows;
-  // (the capacity is below 2^31)
-  auto row_len = [&](int r) { return static_cast<int32_t>(row_keys(p, r, 0)); };
-  auto keys = [&](int r) { return fmaxf(static_cast<float>(row_len(r)), 1.0f); };
-  const int32_t len0 = lane < B ? row_len(lane) : 0;  // rows past the first 64 are read where needed
+  auto keys = [&](int r) { return fmaxf(static_cast<float>(decode_keys(p, r)), 1.0f); };
+  const int32_t len0 = lane < B ? decode_keys(p, lane) : 0;  // rows past the first 64 are read where needed
   const float k0 = lane < B ? fmaxf(static_cast<float>(len0), 1.0f) : 0.0f;
   auto take = [&](int row, int split, int splits) -> DecodeSlot {
-    return {row, split, splits, row < 64 ? __builtin_amdgcn_readlane(len0, row) : row_len(row)};
+    return {row, split, splits, row < 64 ? __builtin_amdgcn_readlane(len0, row) : decode_keys(p, row)};
   };
   float total = k0, most = k0;
   for (int r = lane + 64; r < B; r += 64) {
@@ -697,11 +699,11 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(AttnArgs p) {
     at.splits = __builtin_amdgcn_readfirstlane(at.splits);
     at.keys = __builtin_amdgcn_readfirstlane(at.keys);
   } else {
-    at = {static_cast<int>(blockIdx.z), static_cast<int>(blockIdx.x), p.splits, static_cast<int32_t>(row_keys(p, blockIdx.z, 0))};
+    at = {static_cast<int>(blockIdx.z), static_cast<int>(blockIdx.x), p.splits, decode_keys(p, blockIdx.z)};
   }
   const int64_t qr = at.row, b = qr;
   const int split = at.split;
-  const uint32_t n_keys = static_cast<uint32_t>(max(at.keys, 0));
+  const uint32_t n_keys = static_cast<uint32_t>(at.keys);
   // Slices are whole 32-position steps (a step then never straddles two cache blocks):
   // the slice length is rounded up to 32 and the live split count follows from it,
   // the same in every block of the (row, kv head).
