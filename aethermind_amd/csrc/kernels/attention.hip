@@ -566,7 +566,10 @@ __device__ __forceinline__ float wave_scan(float v) {
 //     kDecSpare blocks beyond it (or a second round of long contexts: 12 rows at 4000-8000
 //     66 us in one, 64 in two) if that ends earlier by the same count of positions.  Split
 //     rows come first.
-// Calls whose rows all may have their most splits in one round have nothing to plan.
+// Calls whose rows all may have their most splits in one round have nothing to plan.  Beyond
+// kDecPlanRows rows the plan's cost in every round of blocks is more than a long row's (250
+// equal rows 163 -> 169 us; 300 rows with one of 16384 225 us without it, 445 with 8 splits
+// for every row): the even split.
 // One row at 16384 positions among 15 at 300 (cold caches, launch included): 113 us with the
 // even split, 50 so, 47 with 8 splits for every row; among 31 201, 56 and 69; 16 rows spread
 // over 50-4000 43, 35 and 41.  Where the split stays even the plan costs 0.2-0.5 us (16 rows
@@ -574,6 +577,7 @@ __device__ __forceinline__ float wave_scan(float v) {
 constexpr float kDecBlockKeys = 400.0f;
 constexpr int kDecSpare = 8;
 constexpr float kDecUneven = 1.33f;
+constexpr int kDecPlanRows = 128;
 struct DecodeSlot {
   int row, split, splits;  // of the row; row < 0: no work
   int32_t keys;
@@ -589,16 +593,22 @@ __device__ __forceinline__ void even_slot(const AttnArgs& p, uint32_t slot, int&
 }
 __device__ __forceinline__ DecodeSlot decode_slot(const AttnArgs& p, int slot, int lane) {
   const int B = p.rows;
-  auto keys = [&](int r) { return fmaxf(static_cast<float>(decode_keys(p, r)), 1.0f); };
-  const int32_t len0 = lane < B ? decode_keys(p, lane) : 0;  // rows past the first 64 are read where needed
-  const float k0 = lane < B ? fmaxf(static_cast<float>(len0), 1.0f) : 0.0f;
+  // a lane's rows: lane, lane + 64, ... (0 past the batch)
+  const int32_t len0 = lane < B ? decode_keys(p, lane) : 0;
+  float k[kDecPlanRows / 64] = {lane < B ? fmaxf(static_cast<float>(len0), 1.0f) : 0.0f};
+#pragma unroll
+  for (int c = 1; c < kDecPlanRows / 64; ++c) {
+    k[c] = 0.0f;
+    if (64 * c < B && 64 * c + lane < B) k[c] = fmaxf(static_cast<float>(decode_keys(p, 64 * c + lane)), 1.0f);
+  }
   auto take = [&](int row, int split, int splits) -> DecodeSlot {
     return {row, split, splits, row < 64 ? __builtin_amdgcn_readlane(len0, row) : decode_keys(p, row)};
   };
-  float total = k0, most = k0;
-  for (int r = lane + 64; r < B; r += 64) {
-    total += keys(r);
-    most = fmaxf(most, keys(r));
+  float total = k[0], most = k[0];
+#pragma unroll
+  for (int c = 1; c < kDecPlanRows / 64; ++c) {
+    total += k[c];
+    most = fmaxf(most, k[c]);
   }
   total = wave_sum(total, lane);
   most = wave_max(most, lane);
@@ -608,16 +618,16 @@ __device__ __forceinline__ DecodeSlot decode_slot(const AttnArgs& p, int slot, i
   const float ideal = B <= p.round ? total / fr : ceilf(fb / fr) * (total / fb + kDecBlockKeys) - kDecBlockKeys;
   float len = 0.0f;  // slice length, 0: the even split
   if (__builtin_expect(even > kDecUneven * fmaxf(ideal, most / fs) + 192.0f, 0)) {
-    auto chunk = [&](int r0) { return r0 == 0 ? k0 : r0 + lane < B ? keys(r0 + lane) : 0.0f; };
     // blocks of slices of l >= most / splits positions: one per row, and one more for each
     // multiple of l below its context
     auto blocks = [&](float l) {
       int n = B;
-      for (int r0 = 0; r0 < B; r0 += 64) {
-        const float k = chunk(r0);
+#pragma unroll
+      for (int c = 0; c < kDecPlanRows / 64; ++c) {
+        if (64 * c >= B) break;
 #pragma unroll
         for (int i = 1; i < kDecMaxSplits; ++i)
-          n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(k > l * static_cast<float>(i)));
+          n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(k[c] > l * static_cast<float>(i)));
       }
       return n;
     };
@@ -645,17 +655,18 @@ __device__ __forceinline__ DecodeSlot decode_slot(const AttnArgs& p, int slot, i
       // rows of several splits, then rows of one
       float at = static_cast<float>(slot);
       for (int pass = 0; pass < 2; ++pass) {
-        for (int r0 = 0; r0 < B; r0 += 64) {
-          const float k = chunk(r0);
-          float n = k > 0.0f ? 1.0f : 0.0f;
 #pragma unroll
-          for (int i = 1; i < kDecMaxSplits; ++i) n += k > len * static_cast<float>(i) ? 1.0f : 0.0f;
+        for (int c = 0; c < kDecPlanRows / 64; ++c) {
+          if (64 * c >= B) break;
+          float n = k[c] > 0.0f ? 1.0f : 0.0f;
+#pragma unroll
+          for (int i = 1; i < kDecMaxSplits; ++i) n += k[c] > len * static_cast<float>(i) ? 1.0f : 0.0f;
           const float mine = (n > 1.0f) == (pass == 0) ? n : 0.0f;
           const float upto = wave_scan(mine), all = lane_value(upto, 63);
           if (at < all) {
             const int i = __builtin_popcountll(__builtin_amdgcn_ballot_w64(upto <= at));
             const float n_row = lane_value(mine, i);
-            return take(r0 + i, static_cast<int>(at - (lane_value(upto, i) - n_row)), static_cast<int>(n_row));
+            return take(64 * c + i, static_cast<int>(at - (lane_value(upto, i) - n_row)), static_cast<int>(n_row));
           }
           at -= all;
         }
@@ -1617,9 +1628,14 @@ extern "C" am_status_code am_gfx950_attention(const am_gfx950_attention_args* a,
       const int64_t even = std::max<int64_t>(1, std::min<int64_t>(p.splits, round / batch));
       const int64_t twice = std::max<int64_t>(1, std::min<int64_t>(p.splits, 2 * round / batch));
       int64_t slots = round;
-      if (even == p.splits) slots = 0;  // as many as a row may have: nothing to plan
-      else if (batch + kDecSpare > round) slots = std::min(batch + kDecSpare, kMaxRows);
-      else if (a->capacity >= kDecLong && 8 * even * pairs < 7 * cus && 8 * twice * pairs >= 14 * cus) slots = 2 * round;
+      if (even == p.splits || batch > kDecPlanRows) {
+        slots = 0;
+        p.splits = static_cast<int32_t>(even);
+      } else if (batch + kDecSpare > round) {
+        slots = batch + kDecSpare;
+      } else if (a->capacity >= kDecLong && 8 * even * pairs < 7 * cus && 8 * twice * pairs >= 14 * cus) {
+        slots = 2 * round;
+      }
       p.rows = static_cast<int32_t>(batch);
       p.round = static_cast<int32_t>(round);
       p.slots = static_cast<int32_t>(slots);

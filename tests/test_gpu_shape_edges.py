@@ -335,7 +335,7 @@ def test_attention_decode_split_rounds(B, hkv, paged):
             assert bool((err <= ref.abs() * 2.0 ** -8 + 2.0 ** -15 * vr.abs().max()).all()), (r, n)
 
 
-@pytest.mark.parametrize("B,hkv", [(16, 8), (24, 8), (32, 8), (100, 8), (9, 24)])
+@pytest.mark.parametrize("B,hkv", [(16, 8), (24, 8), (32, 8), (64, 8), (65, 8), (128, 8), (9, 24)])
 @pytest.mark.parametrize("at", [0, -1])
 def test_attention_decode_one_long_row(B, hkv, at):
     """One long context among short ones keeps its 8 splits whatever the batch (the records
