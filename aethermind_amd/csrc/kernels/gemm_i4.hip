@@ -15,8 +15,8 @@
 //     set by which global chunk each lane fetches: 16-byte chunk c of row r sits at a
 //     slot c ^ f(r) of the row (xsw, wslot), such that the 16 lanes that a 128-bit LDS read
 //     serves at once (rows 0-3 and 12-15 of one k block, rows 4-11 of the next) fall into
-//     distinct banks.  Conflicts counted on the 512-row 8B shapes are 0.3-1.5% of the LDS's
-//     active cycles with bf16 weights, 10-16% with INT4 and 17-20% with INT8, whose 4- and
+//     distinct banks.  Conflicts counted on the 512-row 8B shapes are 0.2-1.5% of the LDS's
+//     active cycles with bf16 weights, 10-16% with INT4 and 16-20% with INT8, whose 4- and
 //     8-byte weight reads have them; half of the cycles before.
 //   * The k loop reads the operands of one 32-value slice while the MFMAs of the slice
 //     before run, also across the barrier between two steps, and converts the next
